@@ -64,7 +64,7 @@ struct Plan {
   bool rec = false;  // layer-sequential path (plh::as_layer_sequential)
   bool fits = true;  // the workgroups of one tile fit the device at once
   bool pad8 = false; // the co-resident tiles are a multiple of 8: a launch may round its grid up to 8 tiles
-  int cap_wgs = 0;   // co-resident workgroups (16-row tiles)
+  int cap_wgs = 0;   // co-resident workgroups of the plan's tile size
 };
 
 Plan make_plan(const plh::Geometry& g, int batch, int cap8, int cap16) {
@@ -74,6 +74,7 @@ Plan make_plan(const plh::Geometry& g, int batch, int cap8, int cap16) {
   if (g.slices == 1 && (long long)g.L * tiles8 <= cap8) {
     p.tile_rows = 8;
     p.chunk_rows = tiles8 * 8;
+    p.cap_wgs = cap8;
     return p;
   }
   // Workgroups per layer of one launch; where the launch is large enough, a multiple of 8 of them
@@ -462,7 +463,13 @@ int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num
     // at H 512 against 9.3 ms at B = 384 (24 tiles).
     // The all-layers sliced kernel likewise rounds its (layer, tile group) groups up to a multiple
     // of 8 where the device holds them (H256 B200: 1.92 ms against 1.47 at B192).
-    a.ntile_grid = g.rec && plan.pad8 ? (a.ntile + 7) / 8 * 8 : a.ntile;
+    // The wavefront kernel's grid likewise, so that the layers of every tile share an XCD: h then goes
+    // from layer to layer through its L2 (C2-like B = 500 and every other tile count not a multiple
+    // of 8 would otherwise write it through to memory).
+    const int ntile8 = (a.ntile + 7) / 8 * 8;
+    const bool wavefront = !g.rec && g.slices == 1;
+    const bool pad = g.rec ? plan.pad8 : wavefront && (long long)g.L * ntile8 <= plan.cap_wgs;
+    a.ntile_grid = pad ? ntile8 : a.ntile;
     const int groups = g.L * a.ntile / a.wg_tiles, groups8 = (groups + 7) / 8 * 8;
     a.groups_grid = g.slices > 1 && !g.rec && groups8 * g.slices <= plan.cap_wgs ? groups8 : groups;
     a.xcd_map = ((g.slices > 1 && !g.rec) ? a.groups_grid % 8 : a.ntile_grid % 8) == 0 ? 1 : 0;

@@ -38,11 +38,14 @@ struct Geometry {
 // The layer-sequential path's padded hidden sizes and the largest hidden size served.
 constexpr int kMaxHidden = 1024;
 
-// u32 words per (layer, tile) counter: the sliced kernels' counters each take a 128-byte line of
-// their own (their workgroups read and update them every few steps, and counters sharing a line
-// serialise those accesses); the wavefront kernels' are adjacent.
-constexpr int kSlicedCounterStride = 32;
-inline int counter_stride(const Geometry& g) { return g.slices > 1 && !g.rec ? kSlicedCounterStride : 1; }
+// u32 words per (layer, tile) counter: each takes a 128-byte line of its own (workgroups read and
+// update them every few steps, and counters sharing a line serialise those accesses).
+constexpr int kCounterStride = 32;
+inline int counter_stride(const Geometry& g) { return g.slices > 1 && !g.rec ? kCounterStride : 1; }
+
+// Steps of the wavefront kernels' hand-off ring (a power of two): h of layers 0..L-2 goes to the layer
+// above step by step, as tagged words in slot t % kHandoffSlots of the ring of its (layer, tile).
+constexpr int kHandoffSlots = 32;
 
 // Fills *g; returns false (with the reason) for geometries the kernels do not implement.
 bool make_geometry(int I, int H, int L, int O, Geometry* g, std::string* why);
@@ -69,11 +72,15 @@ PackedLayout packed_layout(const Geometry& g);
 
 // Workspace of one persistent launch (reused by successive batch chunks); R = rows per tile:
 //   status   u32                                   PLH_STATUS_* bits
-//   counters u32 [L][ntile][counter_stride]       progress published per (layer, tile)
+//   counters u32 [L][ntile][counter_stride]       sliced: progress published per (layer, tile)
 //   xp       f16x8 [ntile][T][g_in0][R]            x in B-fragment order (layer 0 input): group g
 //                                                  holds k = 8g .. 8g+7, the first g_in0 * R
 //                                                  entries of a step's fragment blocks
-//   hseq     f16x8 [L-1][ntile][T][kci][4][R]      h of layers 0..L-2 in B-fragment order
+//   hseq     f16x8 [L-1][ntile][T][kci][4][R]      sliced: h of layers 0..L-2 in B-fragment order;
+//                                                  wavefront kernels: the hand-off rings at its start,
+//                                                  [L-1][ntile][min(T, kHandoffSlots)][HP * R] fp16 words,
+//                                                  and, for T > kHandoffSlots, a 128-byte progress counter
+//                                                  per (layer, tile) behind them, cleared before each launch
 //   xring    u64 [L][ntile][2][HP * 8]             sliced geometries only: per-step exchange of h
 //                                                  among the slices of a (layer, tile), tagged words;
 //            then u32 [L][ntile][16]               the XCD id (+1) of every slice of a group
@@ -105,7 +112,7 @@ struct ForwardArgs {
   const float* wlin;
   const float* blin;
   f16x8_t* xp;                  // packed x, see WorkspaceLayout
-  f16x8_t* hseq;                // inter-layer hand-off, see WorkspaceLayout
+  f16x8_t* hseq;                // inter-layer hand-off (sequence or rings), see WorkspaceLayout
   uint64_t* xring;              // sliced kernels: tagged h exchange ring, zeroed before each launch
   uint32_t* counters;           // [L][ntile][counter_stride] progress published per (layer, tile)
   uint32_t* status;             // PLH_STATUS_* bits
@@ -132,7 +139,8 @@ struct ForwardArgs {
   // layer-sequential kernel (one layer per launch):
   int layer;                    // the layer this launch runs
   int ntile_grid;               // tiles the launch's grid covers (>= ntile: a multiple of 8 where that fits,
-                                // so that every tile's slices share an XCD); the extra ones exit at once
+                                // so that every tile's slices, or layers in the wavefront kernel, share an
+                                // XCD); the extra ones exit at once
   int groups_grid;              // sliced kernels: (layer, tile group) groups the grid covers (>= L ntile /
                                 // wg_tiles, rounded up to 8 the same way; 0: exactly those)
   const _Float16* gates;        // [T * rows_pad][4 HP] blocked: input projection of that layer (no bias), lane order
@@ -148,7 +156,7 @@ hipError_t launch_pack_linear(const Geometry& g, const _Float16* w, const _Float
                               float* blin, hipStream_t s);
 // One launch before each persistent launch: packs this launch's x into xp (g0 8-wide K groups per
 // row and step, zero past I) and clears the status word (if `status`), the counters and ring_words
-// u64 words of the exchange ring.
+// u64 words (an even number) of the exchange ring, or for the wavefront kernels their hand-off rings.
 hipError_t launch_forward_prologue(const Geometry& g, const ForwardArgs& a, uint32_t* status, int g0,
                                    size_t ring_words, hipStream_t s);
 hipError_t launch_zero_u32(uint32_t* p, size_t n, hipStream_t s);

@@ -100,16 +100,16 @@ __global__ void pack_linear_kernel(const _Float16* __restrict__ w, const _Float1
 }
 
 // Forward prologue: x of rows [row0, row_end) into xp (B-fragment order: per tile and step, g0
-// 8-wide K groups of `rows` f16x8, zero past I and past row_end), and the zeroing of up to three
-// u32 ranges (status, counters, exchange ring), in one launch.
+// 8-wide K groups of `rows` f16x8, zero past I and past row_end), and the zeroing of the status and
+// counters (u32) and of the ring (16-byte pieces), in one launch.
 __global__ void forward_prologue_kernel(const _Float16* __restrict__ x, int T, int I, int row0, int row_end,
                                         int ntile, int rows, int g0, f16x8* __restrict__ xp,
                                         uint32_t* __restrict__ z0, size_t n0, uint32_t* __restrict__ z1,
-                                        size_t n1, uint32_t* __restrict__ z2, size_t n2) {
+                                        size_t n1, f16x8* __restrict__ z2, size_t n2) {
   const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e < n0) z0[e] = 0u;
   if (e < n1) z1[e] = 0u;
-  if (e < n2) z2[e] = 0u;
+  if (e < n2) z2[e] = f16x8{};
   const int per = g0 * rows;
   if (e >= (size_t)ntile * T * per) return;
   const int f = (int)(e % per);
@@ -179,12 +179,19 @@ hipError_t launch_forward_prologue(const Geometry& g, const ForwardArgs& a, uint
   const size_t npack = (size_t)a.ntile * a.T * g0 * a.tile_rows;
   const size_t nstat = status ? 1 : 0;
   const size_t nctr = (size_t)g.L * a.ntile * counter_stride(g);
-  const size_t nring = ring_words * 2;  // u64 words as u32
+  // 16-byte pieces of the exchange ring (two u64 words each), or of the hand-off rings and their counters
+  const bool wavefront = !g.rec && g.slices == 1;
+  size_t nring = ring_words / 2;
+  if (wavefront) {
+    nring = (size_t)(g.L - 1) * a.ntile * std::min(a.T, kHandoffSlots) * (g.HP / 8) * a.tile_rows;
+    if (nring && a.T > kHandoffSlots) nring += (size_t)g.L * a.ntile * (kCounterStride / 4);
+  }
+  f16x8* const ring = wavefront ? a.hseq : reinterpret_cast<f16x8*>(a.xring);
   const size_t n = std::max(std::max(npack, nstat), std::max(nctr, nring));
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(forward_prologue_kernel, blocks_for(n, 256), 256, 0, s, a.x, a.T, a.I, a.row0, a.row_end,
                      a.ntile, a.tile_rows, g0, a.xp, status, nstat, a.counters, nctr,
-                     reinterpret_cast<uint32_t*>(a.xring), nring);
+                     ring, nring);
   return hipGetLastError();
 }
 

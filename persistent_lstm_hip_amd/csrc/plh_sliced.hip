@@ -231,7 +231,7 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
   // A (layer, tile) counter counts groups of G steps times the S slices: thread 0 of each slice
   // adds a group once its workgroup's hand-off stores of that group are complete.  Wave 0 reads the
   // upstream counter every step (used a step later) and shares it in LDS.
-  constexpr int CS = kSlicedCounterStride;
+  constexpr int CS = kCounterStride;
   auto up_ctr = [&](int i) -> uint32_t* { return a.counters + ((size_t)(layer - 1) * a.ntile + tile0 + i) * CS; };
   auto my_ctr = [&](int i) -> uint32_t* { return a.counters + ((size_t)layer * a.ntile + tile0 + i) * CS; };
   int pub[NTI];                   // groups of tile i published (thread 0)

@@ -1,0 +1,82 @@
+"""The wavefront kernel's step-by-step hand-off between layers, at the sizes where its ring and its
+unrolled blocks of steps can go wrong: sequences shorter than the pipeline, one step around a block (8) and
+around a lap of the ring (32), several laps; 8- and 16-row tiles; ragged rows; NaN and large frozen h0.
+
+Bound against the oracle's restatement of the device rounding (fp16 h, fp32 sums): a flipped fp16
+rounding of one h moves the final state by a few fp16 ulps of 1 (2^-11 each), so 2e-3."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import make_regressor, make_x, oracle_layers
+from oracle import oracle
+from persistent_lstm_hip_amd import PersistentLSTM
+
+pytestmark = pytest.mark.gpu
+BOUND = 2e-3
+
+
+def _lstm(native):
+    return PersistentLSTM.from_native_module(native.lstm).to("cuda").half().eval()
+
+
+def _oracle(native, x, **kw):
+    return oracle.lstm_forward(x.half().float().numpy(), oracle_layers(native.lstm, half=True), want_seq=True,
+                               numerics="ref_fp16", **kw)
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 7, 8, 9, 11, 12, 13, 31, 32, 33, 40, 63, 65, 100])
+@pytest.mark.parametrize("H,L,B", [(20, 3, 9), (64, 2, 17), (128, 4, 5)])
+def test_lengths_around_the_ring(gpu, H, L, B, T):
+    print(f"[gpu-case] hand-off H={H} L={L} B={B} T={T}", flush=True)
+    native = make_regressor(6, H, L, 3)
+    x = make_x(B, T, 6, seed=T)
+    out, (h, c) = _lstm(native)(x.to("cuda", torch.float16))
+    gpu.check_status(torch.device("cuda"))
+    want = _oracle(native, x)
+    assert np.abs(out.float().cpu().numpy() - want["out_seq"]).max() <= BOUND
+    assert np.abs(h.float().cpu().numpy() - want["h_n"]).max() <= BOUND
+    assert np.abs(c.float().cpu().numpy() - want["c_n"]).max() <= 2 * BOUND
+
+
+@pytest.mark.parametrize("H,L,B,T", [(128, 2, 1100, 41), (60, 4, 40, 70)])
+def test_ragged_rows_and_tiles(gpu, H, L, B, T):
+    """16-row tiles (1100 rows) and 8-row tiles; lengths 0 .. T, rows of length 0 with |h0| up to 3."""
+    print(f"[gpu-case] hand-off ragged H={H} L={L} B={B} T={T}", flush=True)
+    native = make_regressor(5, H, L, 3)
+    x = make_x(B, T, 5, seed=3)
+    g = torch.Generator().manual_seed(4)
+    lengths = torch.randint(0, T + 1, (B,), generator=g)
+    lengths[::7] = 0
+    h0 = (torch.rand(L, B, H, generator=g) * 2 - 1).half()
+    h0[:, lengths == 0] *= 3
+    c0 = torch.randn(L, B, H, generator=g).half()
+    model = _lstm(native)
+    blob = model.packed_blob(torch.device("cuda", torch.cuda.current_device()))
+    res = gpu.forward(blob, (5, H, L, 0), x.to("cuda", torch.float16), lengths=lengths, h0=h0.cuda(), c0=c0.cuda(),
+                      want_out=False, want_seq=True, want_state=True, check_status=True)
+    rows = np.unique(np.r_[0:16, B - 16:B, np.arange(0, B, 7)[:12]])
+    want = _oracle(native, x[rows], lengths=lengths.numpy()[rows], h0=h0.float().numpy()[:, rows],
+                   c0=c0.float().numpy()[:, rows])
+    assert np.abs(res["out_seq"].float().cpu().numpy()[rows] - want["out_seq"]).max() <= BOUND
+    assert np.abs(res["h_n"].float().cpu().numpy()[:, rows] - want["h_n"]).max() <= BOUND
+
+
+@pytest.mark.parametrize("B", [12, 1100])
+def test_nan_stays_in_its_row(gpu, B):
+    """A NaN input: NaN in that row of every layer from that step on, every other row unchanged."""
+    H, L, T, bad, at = 128, 2, 45, 3, 20
+    print(f"[gpu-case] hand-off NaN B={B}", flush=True)
+    model = _lstm(make_regressor(5, H, L, 3))
+    x = make_x(B, T, 5, seed=9).to("cuda", torch.float16)
+    ref = model(x)[0]
+    xn = x.clone()
+    xn[bad, at] = float("nan")
+    got, (h, _) = model(xn)
+    gpu.check_status(torch.device("cuda"))
+    keep = torch.arange(B) != bad
+    assert torch.equal(got[keep], ref[keep])
+    assert torch.equal(got[bad, :at], ref[bad, :at])
+    assert torch.isnan(got[bad, at:]).all() and torch.isnan(h[:, bad]).all()
