@@ -62,6 +62,8 @@ struct Plan {
   int chunk_rows = 16;
   int wg_tiles = 1;  // sliced: 16-row tiles per workgroup
   bool rec = false;  // layer-sequential path (plh::as_layer_sequential)
+  int wide_rows = 0; // wavefront kernel on layer 0's GEMM projections (Geometry::wide_ok): the chunk rows of the
+                     // layer-sequential workspace layout it runs in
   bool fits = true;  // the workgroups of one tile fit the device at once
   bool pad8 = false; // the co-resident tiles are a multiple of 8: a launch may round its grid up to 8 tiles
   int cap_wgs = 0;   // co-resident workgroups of the plan's tile size
@@ -120,8 +122,27 @@ constexpr size_t kMaxSeqWorkspace = (size_t)24 << 30;
 Plan plan_for(const plh::Geometry& g, int batch, int seq_len, bool need_device, hipError_t* err) {
   if (!g.wave_ok) {
     // Padded H 1024, or an input wider than the padded H: only the layer-sequential path exists.
-    Plan q = plan_path(plh::as_layer_sequential(g), batch, need_device, err);
+    const plh::Geometry gr = plh::as_layer_sequential(g);
+    Plan q = plan_path(gr, batch, need_device, err);
     q.rec = true;
+    if (g.wide_ok && *err == hipSuccess) {
+      // Padded H 128: the wavefront kernel, with layer 0's projections from the GEMM, runs every layer
+      // at once without an exchange per step; the layer-sequential kernel runs them one after another,
+      // 1.3 us per step against 0.6-0.8 (I300 H128 L2 B64 T200: 578 -> 180 us).  It runs in the same workspace,
+      // its hand-off rings in the place of the layer sequences: where they do not fit there (more than
+      // three layers on a short sequence), and on a device that cannot hold a tile of all layers, the
+      // layer-sequential path serves the call.
+      Plan p = plan_path(g, batch, need_device, err);
+      if (*err != hipSuccess) return q;
+      p.chunk_rows = std::min(p.chunk_rows, q.chunk_rows);
+      const size_t tiles = (size_t)p.chunk_rows / p.tile_rows;
+      const size_t rings = (size_t)(g.L - 1) * p.chunk_rows * std::min(seq_len, plh::kHandoffSlots) * g.HP * 2 +
+                           (size_t)g.L * tiles * plh::kCounterStride * 4;
+      if (p.fits && rings <= (size_t)2 * seq_len * q.chunk_rows * g.HP * sizeof(_Float16)) {
+        p.wide_rows = q.chunk_rows;
+        return p;
+      }
+    }
     return q;
   }
   const Plan p = plan_path(g, batch, need_device, err);
@@ -364,8 +385,9 @@ int64_t plh_workspace_bytes(int input_size, int hidden_size, int num_layers, int
   }
   hipError_t err = hipSuccess;
   const Plan p = plan_for(g, batch, seq_len, false, &err);
-  if (p.rec) g = plh::as_layer_sequential(g);
-  return (int64_t)plh::workspace_layout(g, seq_len, p.chunk_rows, p.tile_rows).total;
+  if (p.rec || p.wide_rows) g = plh::as_layer_sequential(g);
+  return (int64_t)plh::workspace_layout(g, seq_len, p.wide_rows ? p.wide_rows : p.chunk_rows,
+                                        p.wide_rows ? 16 : p.tile_rows).total;
 }
 
 int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num_layers, int output_size,
@@ -394,7 +416,9 @@ int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num
                                          " workgroups of one batch tile co-resident (layers = " +
                                          std::to_string(g.L) + ")");
   const int chunk_rows = plan.chunk_rows;
-  const plh::WorkspaceLayout w = plh::workspace_layout(g, seq_len, chunk_rows, plan.tile_rows);
+  const plh::WorkspaceLayout w =
+      plan.wide_rows ? plh::workspace_layout(plh::as_layer_sequential(g), seq_len, plan.wide_rows, 16)
+                     : plh::workspace_layout(g, seq_len, chunk_rows, plan.tile_rows);
   if (workspace_bytes < (int64_t)w.total)
     return fail(PLH_ERR_INVALID, "workspace smaller than plh_workspace_bytes()");
 
@@ -446,7 +470,7 @@ int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num
 
   KernelTiming& tm = timing();
   const bool timed = tm.used * 2 < (int)tm.ev.size();
-  const int cus = g.rec ? device_cus(&err) : 0;
+  const int cus = g.rec || plan.wide_rows ? device_cus(&err) : 0;
   if (err != hipSuccess) return fail_hip(err, "device query");
   for (int row0 = 0; row0 < batch; row0 += chunk_rows) {
     const int rows = std::min(chunk_rows, batch - row0);
@@ -519,13 +543,29 @@ int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num
       a.wx0 = nullptr;
       continue;
     }
-    // x of this launch's rows into xp; status (first launch), counters and, when sliced, the
-    // exchange ring (tags restart at 1) cleared: one launch ahead of the persistent one
-    err = plh::launch_forward_prologue(g, a, row0 == 0 ? status : nullptr, g.g_in0, w.xring_words, s);
+    // x of this launch's rows into xp; status (first launch), counters and rings cleared (tags restart): one
+    // launch ahead of the persistent one
+    if (plan.wide_rows) {
+      a.wpack = (const _Float16*)(pk + p.wrec);
+      a.hseq = (plh::f16x8_t*)(ws + w.xs);
+      a.gates = (const _Float16*)(ws + w.gates);
+      a.wih_up = (const _Float16*)(pk + p.wih) + (size_t)4 * g.HP * g.kp0;
+    }
+    err = plh::launch_forward_prologue(g, a, row0 == 0 ? status : nullptr, plan.wide_rows ? 0 : g.g_in0,
+                                       w.xring_words, s);
     if (err != hipSuccess) return fail_hip(err, "forward prologue");
     if (timed && row0 == 0) {
       err = hipEventRecord(tm.ev[2 * tm.used], s);
       if (err != hipSuccess) return fail_hip(err, "timing event");
+    }
+    if (plan.wide_rows) {
+      // layer 0's projections of every step and row of this launch (a whole number of 16-row blocks)
+      err = plh::launch_rec_input(g, a, (_Float16*)(ws + w.xin), g.kp0, s);
+      if (err != hipSuccess) return fail_hip(err, "input transpose");
+      err = plh::launch_proj_gemm((const _Float16*)(ws + w.xin), g.kp0, (const _Float16*)(pk + p.wih), g.kp0,
+                                  (_Float16*)(ws + w.gates), 4 * g.HP,
+                                  ((long long)seq_len * a.rows_pad + 15) / 16 * 16, 4 * g.HP, true, cus, s);
+      if (err != hipSuccess) return fail_hip(err, "input projection GEMM launch");
     }
     err = plh::launch_recurrent(g, a, s);
     if (err != hipSuccess) return fail_hip(err, "persistent LSTM launch");

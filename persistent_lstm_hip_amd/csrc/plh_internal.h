@@ -22,6 +22,8 @@ struct Geometry {
   int slices;  // workgroups per (layer, tile): 1, 4 (HP = 256), 16 (HP = 512); on the layer-sequential
                // path Rec<HP>::kS (2, 4, 8, 32)
   int wave_ok;  // the all-layers kernels serve this geometry (HP <= 512 and I <= HP)
+  int wide_ok;  // ... or the wavefront kernel does, with layer 0's projections from the GEMM (HP = 128 < I);
+                // its weights are those of the layer-sequential path
   int rec_ok;  // the layer-sequential path serves it (HP >= 512, or I > HP): its weights are packed too
   int rec;     // this forward runs layer by layer: input projection as a GEMM, recurrent kernel
                // holding W_hh alone (make_geometry leaves 0; as_layer_sequential sets it)
@@ -144,6 +146,8 @@ struct ForwardArgs {
   int groups_grid;              // sliced kernels: (layer, tile group) groups the grid covers (>= L ntile /
                                 // wg_tiles, rounded up to 8 the same way; 0: exactly those)
   const _Float16* gates;        // [T * rows_pad][4 HP] blocked: input projection of that layer (no bias), lane order
+                                // (wavefront kernel: of layer 0, where the input is wider than HP; else null)
+  const _Float16* wih_up;       // wavefront kernel with gates: W_ih of layers 1.., [4 HP][HP] each, rows in lane order
   _Float16* hout;               // [T * rows_pad][HP] blocked: its h sequence, the next layer's input (null: last layer)
   const _Float16* wx0;          // rec_x0, layer 0: W_ih fragments of the in-kernel projection (x from xp)
 };
@@ -163,9 +167,10 @@ hipError_t launch_zero_u32(uint32_t* p, size_t n, hipStream_t s);
 hipError_t launch_repeat_first_row(const _Float16* in, _Float16* out, int rows, int cols, hipStream_t s);
 
 // Persistent kernels (device function pointers for hipLaunchKernel), nullptr if no variant
-// exists: the wavefront kernel for padded H <= 128 and 8- or 16-row tiles (plh_wavefront.hip), the
+// exists: the wavefront kernel for padded H <= 128 and 8- or 16-row tiles (plh_wavefront.hip; wide: on the
+// projections of an input wider than the padded H, 128 only), the
 // sliced kernel for padded H 256 / 512 with 1 or 2 tiles per workgroup (plh_sliced.hip).
-const void* wavefront_kernel(int HP, int tile_rows, bool ragged);
+const void* wavefront_kernel(int HP, int tile_rows, bool ragged, bool wide);
 const void* sliced_kernel(int HP, int wg_tiles);
 
 // Co-resident workgroups of the persistent kernel on the current device (0 with *err set on error).

@@ -34,6 +34,7 @@ bool make_geometry(int I, int H, int L, int O, Geometry* g, std::string* why) {
   g->O = O;
   g->HP = HP;
   g->wave_ok = (HP <= 512 && I <= HP) ? 1 : 0;
+  g->wide_ok = (HP == 128 && I > HP) ? 1 : 0;
   g->rec_ok = (HP >= 512 || I > HP) ? 1 : 0;
   g->rec = 0;
   g->slices = HP == 256 ? Sliced<256>::kS : HP == 512 ? Sliced<512>::kS : 1;
@@ -117,7 +118,7 @@ static const void* recurrent_kernel(const Geometry& g, int tile_rows, bool ragge
                                     bool x0 = false) {
   if (g.rec) return tile_rows == 16 && wg_tiles == 1 ? rec_kernel(g.HP, x0) : nullptr;
   if (g.slices > 1) return tile_rows == 16 ? sliced_kernel(g.HP, wg_tiles) : nullptr;
-  return wavefront_kernel(g.HP, tile_rows, ragged);
+  return wavefront_kernel(g.HP, tile_rows, ragged, g.wide_ok != 0);
 }
 
 int recurrent_capacity(const Geometry& g, int tile_rows, hipError_t* err) {

@@ -178,9 +178,9 @@ hipError_t launch_forward_prologue(const Geometry& g, const ForwardArgs& a, uint
                                    size_t ring_words, hipStream_t s) {
   const size_t npack = (size_t)a.ntile * a.T * g0 * a.tile_rows;
   const size_t nstat = status ? 1 : 0;
-  const size_t nctr = (size_t)g.L * a.ntile * counter_stride(g);
   // 16-byte pieces of the exchange ring (two u64 words each), or of the hand-off rings and their counters
   const bool wavefront = !g.rec && g.slices == 1;
+  const size_t nctr = wavefront ? 0 : (size_t)g.L * a.ntile * counter_stride(g);
   size_t nring = ring_words / 2;
   if (wavefront) {
     nring = (size_t)(g.L - 1) * a.ntile * std::min(a.T, kHandoffSlots) * (g.HP / 8) * a.tile_rows;

@@ -104,21 +104,24 @@ __device__ __forceinline__ bool handoff_special(uint32_t w) {
   return !(__builtin_fabsf(__builtin_bit_cast(float, w)) <= __builtin_bit_cast(float, 0x3C00FFFFu));
 }
 
-// Where a layer's step input comes from: the layer below (tagged words), or x with one K chunk
-// (I <= 32, so the input MFMAs on the other, all-zero chunks are skipped) or with all of them.
-enum class Src { kUp, kX1, kXn };
+// Where a layer's step input comes from: the layer below (tagged words), x with one K chunk (I <= 32, so
+// the input MFMAs on the other, all-zero chunks are skipped) or with all of them, or, for an input wider
+// than the padded hidden size, its projection x_t W_ih^T from the projection GEMM (padded H 128).
+enum class Src { kUp, kX1, kXn, kGates };
 
 // The persistent layer-wavefront recurrence of one (layer, tile).  Template: padded hidden size HP,
 // batch rows per workgroup ROWS (16, or 8 with the MFMA's B columns 8..15 duplicating rows 0..7 so
 // each lane evaluates two (unit, row) pairs instead of four), RAGGED: rows may end before the
 // tile's last step (lengths given; without it every row is live at every step and the
-// state-freezing selects are compiled out), the step input's source, and DOWN: a layer above takes h.
-template <int HP, int ROWS, bool RAGGED, Src SRC, bool DOWN>
+// state-freezing selects are compiled out), WIDE: the model's
+// input is wider than HP, the step input's source, and DOWN: a layer above takes h.
+template <int HP, int ROWS, bool RAGGED, bool WIDE, Src SRC, bool DOWN>
 __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLds<HP, ROWS>& lds, int layer, int tile) {
   using C = Tile<HP, ROWS>;
   constexpr int KCI = C::kKci, KCR = C::kKcr, KC = C::kKc, NT = C::kThreads, FV = C::kFragVec;
   constexpr bool UP = SRC == Src::kUp;
-  constexpr int KIN = SRC == Src::kX1 ? 1 : KCI;  // input-part K chunks with MFMA work
+  constexpr bool GATES = SRC == Src::kGates;
+  constexpr int KIN = SRC == Src::kX1 ? 1 : GATES ? 0 : KCI;  // input-part K chunks with MFMA work
   constexpr int UPL = C::kUpl, NW = C::kNw;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -146,12 +149,31 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
 
   // Resident weights: A fragments of [W_ih | W_hh] rows for this wave's 16 units, 4 gates.
   f16x8 w[KC][4];
-  {
+  if constexpr (!WIDE) {
     const f16x8* wp = reinterpret_cast<const f16x8*>(a.wpack) + ((size_t)(layer * C::kWaves + wave) * KC * 4) * 64 + lane;
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc)
 #pragma unroll
       for (int q = 0; q < 4; ++q) w[kc][q] = (kc < KIN || kc >= KCI) ? wp[(kc * 4 + q) * 64] : f16x8{};
+  } else {
+    // Models with an input wider than the padded H are packed for the layer-sequential path only: gather
+    // the same fragments (row: unit u of gate q, k: 8 kg .. + 7 of the chunk) from its W_hh fragments
+    // (pack_rec_kernel: slice u / 64, wave u / 8 % 8, tile u / 4 % 2, row 4 (u % 4) + q) and from its W_ih
+    // rows in lane order (rec_lane_column).
+    const int u = wave * 16 + n;
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        w[kc][q] = f16x8{};
+        if (kc >= KCI)
+          w[kc][q] = reinterpret_cast<const f16x8*>(
+              a.wpack)[((((size_t)layer * 16 + (u >> 3)) * KCR + kc - KCI) * 2 + ((u >> 2) & 1)) * 64 + kg * 16 + (u & 3) * 4 + q];
+        else if (UP)
+          w[kc][q] = *reinterpret_cast<const f16x8*>(
+              a.wih_up + ((size_t)(layer - 1) * 4 * HP + ((u >> 3) * 4 + (u & 3)) * 8 + 2 * q + ((u >> 2) & 1)) * HP +
+              kc * 32 + kg * 8);
+      }
   }
   // D rows of this lane: units u0 .. u0+3 of row n; it evaluates UPL of them, starting at uo.
   const int u0 = wave * 16 + kg * 4;
@@ -302,7 +324,7 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
   // A step's source holds the first `per` f16x8 of its fragment blocks (the g_in0 8-wide K groups of x);
   // the rest are written as zeros.
   constexpr int XS = KIN * FV;  // f16x8 per step in LDS
-  constexpr int RN = (kBlock * XS + NT - 1) / NT;
+  constexpr int RN = GATES ? 1 : (kBlock * XS + NT - 1) / NT;
   const int per = a.g_in0 * ROWS;
   const f16x8* const xsrc = a.xp + (size_t)tile * a.T * per;
   f16x8 R[RN];
@@ -310,7 +332,7 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
 #pragma unroll
     for (int i = 0; i < RN; ++i) {
       const int p = (int)threadIdx.x + i * NT;
-      const int st = p / XS, e = p % XS;
+      const int st = p / (XS ? XS : 1), e = p % (XS ? XS : 1);
       const size_t s = (size_t)clamp_step(k * kBlock + (st < kBlock ? st : kBlock - 1));
       R[i] = xsrc[s * per + (e < per ? e : per - 1)];
     }
@@ -320,8 +342,31 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
 #pragma unroll
     for (int i = 0; i < RN; ++i) {
       const int p = (int)threadIdx.x + i * NT;
-      if (p < kBlock * XS) rb[p] = p % XS < per ? R[i] : f16x8{};
+      if (p < kBlock * XS) rb[p] = p % (XS ? XS : 1) < per ? R[i] : f16x8{};
     }
+  };
+
+  // ---- layer 0 with a wide input: the projections, loaded two steps before they are added ----
+  // Step t's row of this lane is row t rows_pad + tile ROWS + r of the blocked [.. x 4 HP] projections; the 16
+  // bytes of column group (u / 8, u % 4) hold the four gates of units u and u + 4, alternating.
+  const f16x8* const gsrc = reinterpret_cast<const f16x8*>(a.gates);
+  f16x8 gates[2][UPL];
+  auto load_gates = [&](int t, f16x8 (&g)[UPL]) __attribute__((always_inline)) {
+    const size_t row = (size_t)clamp_step(t) * a.rows_pad + tile * ROWS + r;
+    const f16x8* src = gsrc + ((row >> 4) * (4 * HP / 32) + (uo >> 3)) * 64 + (uo & 3) * 16 + (row & 15);
+#pragma unroll
+    for (int j = 0; j < UPL; ++j) g[j] = src[j * 16];
+  };
+  // acc = bias + the projections (8-row tiles: both candidates of a lane's pair, as it evaluates one)
+  const bool upper = ((uo >> 2) & 1) != 0;
+  auto add_gates = [&](const f16x8 (&g)[UPL], f32x4 (&acc)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f16x8 v = g[j % UPL];
+        acc[q][j] = bias[q][j] + (float)(upper ? v[2 * q + 1] : v[2 * q]);
+      }
   };
   // LDS slot of step t's input.
   auto xin_at = [&](int t) -> f16x8* { return UP ? lds.xin + (t & 1) * XS : lds.xin + (t & (2 * kBlock - 1)) * XS; };
@@ -381,7 +426,7 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
         wait_vmem_all();
         put_word(check_word(handoff_tag(sc), slot_of(sc), words[s]), xin_at(s));
       }
-    } else {
+    } else if constexpr (!GATES) {
       load_block(0);
       wait_vmem_all();
       store_block(0);
@@ -400,9 +445,15 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
     }
   }
   __syncthreads();
-  if (Tt > 0) {
+  if (GATES && Tt > 0) {
+    load_gates(0, gates[0]);
+    wait_vmem_all();
+    add_gates(gates[0], acc_next);
+    load_gates(1, gates[1]);
+    load_gates(2, gates[0]);
+  } else if (Tt > 0) {
     const f16x8* xr = xin_at(0) + fl;
-    f16x8 xv[KIN];
+    f16x8 xv[KIN ? KIN : 1];
 #pragma unroll
     for (int kc = 0; kc < KIN; ++kc) xv[kc] = xr[kc * FV];
 #pragma unroll
@@ -440,7 +491,7 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
     __builtin_amdgcn_sched_barrier(0);
     wvec x2 = {};
     if constexpr (UP) x2 = check_word(FULL ? block_tag(2) : handoff_tag(s2), FULL ? block_slot(2) : slot_of(s2), words[P]);
-    if constexpr (!UP) {
+    if constexpr (!UP && !GATES) {
       if (s == 2) {
         // (also ends what is outstanding: without it the compiler keeps the block loads "possibly
         // outstanding", their consumers being lane-conditional)
@@ -473,12 +524,17 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
     // would otherwise queue all VALU work behind a burst of MFMAs).
     const f16x8* xr = (UP ? lds.xin + (P ^ 1) * XS
                           : lds.xin + ((s + 1 < kBlock ? (k & 1) * kBlock + s + 1 : ((k + 1) & 1) * kBlock)) * XS) + fl;
-    f16x8 xv[KIN];
+    f16x8 xv[KIN ? KIN : 1];
 #pragma unroll
     for (int kc = 0; kc < KIN; ++kc) xv[kc] = xr[kc * FV];
     if constexpr (UP) put_word(x2, lds.xin + P * XS);  // (after the reads, which then move up among the MFMAs)
+    if constexpr (GATES) {
+      add_gates(gates[P ^ 1], acc_next);  // step t + 1's
+      load_gates(t + 3, gates[P ^ 1]);
+    } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) acc_next[q] = bias[q];
+      for (int q = 0; q < 4; ++q) acc_next[q] = bias[q];
+    }
     const bool live = t < len;
     auto input_mfma = [&](int m) __attribute__((always_inline)) {
       const int kc = m / 4, q = m % 4;
@@ -654,7 +710,7 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
 // At least two waves per SIMD in the bounds keep a wave within 256 registers, where MFMAs take and leave
 // their accumulators in VGPRs; with one (what 128- and 256-thread workgroups default to) they went to
 // AGPRs, and every step copied its 16 gate sums back.
-template <int HP, int ROWS, bool RAGGED>
+template <int HP, int ROWS, bool RAGGED, bool WIDE>
 __global__ void __launch_bounds__(HP / 16 * 64, 2)
 lstm_wavefront_kernel(ForwardArgs a) {
   __shared__ WavefrontLds<HP, ROWS> lds;
@@ -664,33 +720,39 @@ lstm_wavefront_kernel(ForwardArgs a) {
   auto body = [&](auto src) __attribute__((always_inline)) {
     constexpr Src SRC = decltype(src)::value;
     if (layer + 1 < a.L)
-      wavefront_body<HP, ROWS, RAGGED, SRC, true>(a, lds, layer, tile);
+      wavefront_body<HP, ROWS, RAGGED, WIDE, SRC, true>(a, lds, layer, tile);
     else
-      wavefront_body<HP, ROWS, RAGGED, SRC, false>(a, lds, layer, tile);
+      wavefront_body<HP, ROWS, RAGGED, WIDE, SRC, false>(a, lds, layer, tile);
   };
-  if (layer > 0)
+  if (layer > 0) {
     body(std::integral_constant<Src, Src::kUp>());
-  else if (a.g_in0 <= 4)
+  } else if constexpr (WIDE) {
+    body(std::integral_constant<Src, Src::kGates>());
+  } else if (a.g_in0 <= 4) {
     body(std::integral_constant<Src, Src::kX1>());
-  else
+  } else {
     body(std::integral_constant<Src, Src::kXn>());
+  }
 }
 
 }  // namespace
 
 template <int ROWS, bool RAGGED>
-static const void* wavefront_kernel_rows(int HP) {
+static const void* wavefront_kernel_rows(int HP, bool wide) {
+  if (wide) return HP == 128 ? reinterpret_cast<const void*>(&lstm_wavefront_kernel<128, ROWS, RAGGED, true>) : nullptr;
   switch (HP) {
-    case 32: return reinterpret_cast<const void*>(&lstm_wavefront_kernel<32, ROWS, RAGGED>);
-    case 64: return reinterpret_cast<const void*>(&lstm_wavefront_kernel<64, ROWS, RAGGED>);
-    case 128: return reinterpret_cast<const void*>(&lstm_wavefront_kernel<128, ROWS, RAGGED>);
+    case 32: return reinterpret_cast<const void*>(&lstm_wavefront_kernel<32, ROWS, RAGGED, false>);
+    case 64: return reinterpret_cast<const void*>(&lstm_wavefront_kernel<64, ROWS, RAGGED, false>);
+    case 128: return reinterpret_cast<const void*>(&lstm_wavefront_kernel<128, ROWS, RAGGED, false>);
     default: return nullptr;
   }
 }
 
-const void* wavefront_kernel(int HP, int tile_rows, bool ragged) {
-  if (tile_rows == 8) return ragged ? wavefront_kernel_rows<8, true>(HP) : wavefront_kernel_rows<8, false>(HP);
-  if (tile_rows == 16) return ragged ? wavefront_kernel_rows<16, true>(HP) : wavefront_kernel_rows<16, false>(HP);
+const void* wavefront_kernel(int HP, int tile_rows, bool ragged, bool wide) {
+  if (tile_rows == 8)
+    return ragged ? wavefront_kernel_rows<8, true>(HP, wide) : wavefront_kernel_rows<8, false>(HP, wide);
+  if (tile_rows == 16)
+    return ragged ? wavefront_kernel_rows<16, true>(HP, wide) : wavefront_kernel_rows<16, false>(HP, wide);
   return nullptr;
 }
 

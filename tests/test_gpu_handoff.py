@@ -80,3 +80,29 @@ def test_nan_stays_in_its_row(gpu, B):
     assert torch.equal(got[keep], ref[keep])
     assert torch.equal(got[bad, :at], ref[bad, :at])
     assert torch.isnan(got[bad, at:]).all() and torch.isnan(h[:, bad]).all()
+
+
+@pytest.mark.parametrize("I,H,L,B,T", [
+    (129, 128, 1, 3, 1),      # one layer, one step, half a 16-row block
+    (300, 60, 3, 17, 33),     # three 8-row tiles: T * rows not a multiple of 16
+    (200, 100, 2, 1100, 4),   # 16-row tiles
+    (150, 128, 4, 9, 47),     # four layers: rings larger than the layer sequences' place, layer by layer
+    (150, 128, 4, 9, 48),     # ... and just fitting it
+    (140, 120, 2, 2100, 3),   # more rows than one launch holds
+])
+def test_wide_inputs(gpu, I, H, L, B, T):
+    """Inputs wider than the padded hidden size: layer 0's projections are rounded to fp16 (half an ulp of
+    a pre-activation below 4 is 2^-10, and a gate moves by at most that), on top of BOUND."""
+    print(f"[gpu-case] wide I={I} H={H} L={L} B={B} T={T}", flush=True)
+    native = make_regressor(I, H, L, 3)
+    x = make_x(B, T, I, seed=7)
+    lengths = torch.randint(0, T + 1, (B,), generator=torch.Generator().manual_seed(5))
+    model = _lstm(native)
+    blob = model.packed_blob(torch.device("cuda", torch.cuda.current_device()))
+    rows = np.unique(np.r_[0:min(B, 9), max(0, B - 9):B])
+    for lens in (None, lengths):
+        res = gpu.forward(blob, (I, H, L, 0), x.to("cuda", torch.float16), lengths=lens, want_out=False, want_seq=True,
+                          want_state=True, check_status=True)
+        want = _oracle(native, x[rows], lengths=None if lens is None else lens.numpy()[rows])
+        assert np.abs(res["out_seq"].float().cpu().numpy()[rows] - want["out_seq"]).max() <= 2 * BOUND
+        assert np.abs(res["h_n"].float().cpu().numpy()[:, rows] - want["h_n"]).max() <= 2 * BOUND
