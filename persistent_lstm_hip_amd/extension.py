@@ -84,15 +84,38 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+def _index(device: torch.device) -> int:
+    return device.index if device.index is not None else torch.cuda.current_device()
+
+
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The handle of the device's current stream (without the Stream object around it)."""
+    return torch._C._cuda_getCurrentRawStream(_index(device))
 
 
 def _device_key(device: torch.device) -> tuple:
     """(type, index, current stream) with the index resolved, so "cuda" and "cuda:0" name one device."""
     device = torch.device(device)
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    return (device.type, index, _stream(torch.device(device.type, index)))
+    index = _index(device)
+    return (device.type, index, torch._C._cuda_getCurrentRawStream(index))
+
+
+class _on_device:
+    """torch.cuda.device(device) that does nothing when it is already the current device."""
+
+    __slots__ = ("index", "prev")
+
+    def __init__(self, device: torch.device):
+        self.index = _index(device)
+
+    def __enter__(self) -> None:
+        self.prev = torch.cuda.current_device()
+        if self.prev != self.index:
+            torch.cuda.set_device(self.index)
+
+    def __exit__(self, *exc) -> None:
+        if self.prev != self.index:
+            torch.cuda.set_device(self.prev)
 
 
 class NativeLibrary:
@@ -179,7 +202,7 @@ class NativeLibrary:
         lw, lb = half(lin_w), half(lin_b)
         nbytes = self.packed_bytes(I, H, L, O)
         packed = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        with torch.cuda.device(device):
+        with _on_device(device):
             rc = self.lib.plh_pack_regressor(
                 I, H, L, O, a_wih, a_whh, a_bih, a_bhh, _ptr(lw), _ptr(lb), packed.data_ptr(), nbytes,
                 _stream(device),
@@ -237,9 +260,8 @@ class NativeLibrary:
             raise ValueError("x must be a floating-point tensor")
         device = x.device
         B, T = int(x.size(0)), int(x.size(1))
-        xh = x.to(torch.float16).contiguous()
-        opts = dict(device=device, dtype=torch.float16)
-        given = dict(outputs or {})
+        xh = (x if x.dtype is torch.float16 else x.to(torch.float16)).contiguous()
+        given = dict(outputs) if outputs else {}
 
         def buf(name, shape, dtype=torch.float16):
             t = given.pop(name, None)
@@ -277,8 +299,8 @@ class NativeLibrary:
                 continue
             if tuple(s.shape) != (L, B, H):
                 raise ValueError(f"initial states must be [{L}, {B}, {H}]")
-            states.append(s.to(**opts).contiguous())
-        probes = sorted(set(int(p) for p in (probe_steps or ())))
+            states.append(s.to(device=device, dtype=torch.float16).contiguous())
+        probes = sorted(set(int(p) for p in probe_steps)) if probe_steps is not None else []
         if probes and (probes[0] < 1 or probes[-1] > T):
             raise ValueError(f"probe steps must lie in [1, {T}]")
         P = len(probes)
@@ -289,7 +311,7 @@ class NativeLibrary:
             raise ValueError(f"outputs given for ones not requested: {sorted(given)}")
         if packed.device != device:
             raise ValueError("packed weights and x must be on the same device")
-        with torch.cuda.device(device):
+        with _on_device(device):
             nws = self.workspace_bytes(I, H, L, O, B, T)
             ws = self.workspace(device, nws)
             rc = self.lib.plh_forward(
@@ -317,7 +339,7 @@ class NativeLibrary:
         if ws is None:
             return 0
         st = ctypes.c_uint32(0)
-        with torch.cuda.device(device):
+        with _on_device(device):
             self._check(self.lib.plh_status(ws.data_ptr(), ctypes.byref(st), _stream(device)), "plh_status")
         return int(st.value)
 
@@ -391,7 +413,7 @@ class NativeLibrary:
               or (blocked and not out.is_contiguous())):
             raise ValueError("out must be a float16 [rows, cols] tensor with unit column stride (blocked: contiguous)")
         ldo = cols if (blocked or rows <= 1) else int(out.stride(0))
-        with torch.cuda.device(x.device):
+        with _on_device(x.device):
             rc = self.lib.plh_input_projection(x.data_ptr(), ldx, w.data_ptr(), k, out.data_ptr(), ldo, rows, cols,
                                                1 if blocked else 0, _stream(x.device))
         self._check(rc, "plh_input_projection")
@@ -420,7 +442,7 @@ class NativeLibrary:
         inp = inp.contiguous()
         cols = int(inp.size(1))
         out = torch.empty((int(output_batch_size), cols), dtype=inp.dtype, device=inp.device)
-        with torch.cuda.device(inp.device):
+        with _on_device(inp.device):
             rc = self.lib.plh_repeat_first_row(inp.data_ptr(), out.data_ptr(), int(output_batch_size), cols,
                                                _stream(inp.device))
         self._check(rc, "plh_repeat_first_row")

@@ -43,6 +43,10 @@ def _debug() -> bool:
     return os.environ.get("PERSISTENT_LSTM_HIP_DEBUG", "0") == "1"
 
 
+def _uniform_mode() -> str:
+    return os.environ.get("PERSISTENT_LSTM_HIP_UNIFORM_BATCH", "auto").strip().lower()
+
+
 def _check_after(ext, device: torch.device) -> None:
     """With PERSISTENT_LSTM_HIP_CHECK_STATUS=1, every module forward synchronises its stream and
     raises RuntimeError if the kernel reported a failure (a timed-out wait between workgroups).
@@ -94,25 +98,26 @@ class NativeModuleFallback(nn.Module):
 
 class _TensorSetKey:
     """Identity of a list of tensors for a cache: the same live objects (weak references, so an id
-    reused by a later object never matches) with unchanged version counters, storage, dtype and
-    device."""
+    reused by a later object never matches) with unchanged version counters, addresses, shapes and
+    dtypes (an address also names its device: the devices of a process share one address space).
+    Checked on every forward, so attribute by attribute rather than through a tuple per tensor."""
 
     def __init__(self, tensors: Sequence[Optional[torch.Tensor]]):
-        self._refs = [None if t is None else weakref.ref(t) for t in tensors]
-        self._sig = self.signature(tensors)
-
-    @staticmethod
-    def signature(tensors: Sequence[Optional[torch.Tensor]]) -> tuple:
-        return tuple(None if t is None else (t._version, t.data_ptr(), tuple(t.shape), str(t.dtype), t.device.type,
-                                             t.device.index) for t in tensors)
+        self._entries = [None if t is None else (weakref.ref(t), t._version, t.data_ptr(), t.shape, t.dtype)
+                         for t in tensors]
 
     def matches(self, tensors: Sequence[Optional[torch.Tensor]]) -> bool:
-        if len(tensors) != len(self._refs):
+        entries = self._entries
+        if len(tensors) != len(entries):
             return False
-        for r, t in zip(self._refs, tensors):
-            if (r is None) != (t is None) or (r is not None and r() is not t):
+        for e, t in zip(entries, tensors):
+            if e is None or t is None:
+                if e is not t:
+                    return False
+            elif (e[0]() is not t or t._version != e[1] or t.data_ptr() != e[2] or t.shape != e[3]
+                  or t.dtype is not e[4]):
                 return False
-        return self.signature(tensors) == self._sig
+        return True
 
 
 class PersistentLSTM(nn.Module):
@@ -164,11 +169,11 @@ class PersistentLSTM(nn.Module):
 
     def packed_blob(self, device: torch.device, linear: Optional[nn.Linear] = None) -> torch.Tensor:
         """The device-resident packed weights (re-packed when a parameter or its version changes)."""
-        params = []
-        for l in range(self.num_layers):
-            params.extend(self.layer_params(l))
+        params = list(self._parameters.values())
+        if len(params) != (4 if self.bias else 2) * self.num_layers:  # e.g. a parametrized weight
+            params = [p for l in range(self.num_layers) for p in self.layer_params(l)]
         if linear is not None:
-            params.extend([linear.weight, linear.bias])
+            params += (linear.weight, linear.bias)
         dev = (device.type, device.index)
         if self._pack_blob is None or self._pack_device != dev or not self._pack_key.matches(params):
             ext = require_extension()
@@ -261,7 +266,7 @@ class PersistentLSTMRegressor(nn.Module):
         which would broadcast row 0 of a non-uniform input.  A weak reference cannot: once the tensor
         it saw is freed it resolves to None.  Writes that bypass the version counter (`.data`, raw
         pointers) are not seen, as in the reference."""
-        mode = os.environ.get("PERSISTENT_LSTM_HIP_UNIFORM_BATCH", "auto").strip().lower()
+        mode = _uniform_mode()
         if mode in _OFF or x.dim() != 3 or x.size(0) <= 1:
             return False
         if mode in _ON:
@@ -290,17 +295,18 @@ class PersistentLSTMRegressor(nn.Module):
         ext = require_extension()
         self._check_input(x)
         blob = self.lstm.packed_blob(x.device, self.linear)
+        dims = self.dims()
         batch = int(x.size(0))
         uniform = self._should_use_uniform_batch_fast_path(x)
-        if _debug() and not self._debug_reported:
+        if not self._debug_reported and _debug():
             print(f"persistent_lstm_hip_amd debug: backend={BACKEND_NAME}, batch={batch}, "
-                  f"seq_len={int(x.size(1))}, dims={self.dims()}, uniform_batch_fast_path={uniform}")
+                  f"seq_len={int(x.size(1))}, dims={dims}, uniform_batch_fast_path={uniform}")
             self._debug_reported = True
         if uniform:
-            row = ext.forward(blob, self.dims(), x.narrow(0, 0, 1))["out"]
+            row = ext.forward(blob, dims, x.narrow(0, 0, 1))["out"]
             out = ext.repeat_first_row(row, batch)
         else:
-            out = ext.forward(blob, self.dims(), x)["out"]
+            out = ext.forward(blob, dims, x)["out"]
         _check_after(ext, x.device)
         return out if x.dtype == torch.float16 else out.to(x.dtype)
 
