@@ -115,6 +115,19 @@ int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num
                 int64_t workspace_bytes, void* stream);
 
 /*
+ * plh_forward of the head alone ([batch, O], full-length rows, zero initial state) for a batch whose rows
+ * may all be equal, which the reference's dispatcher looks for on the host before every forward
+ * (model.py:493-520) to run one row of it (model.py:628-645).  Where plh_detects_uniform() is 1 the forward
+ * finds out on the device while it packs x, without a host synchronisation, and a batch of equal rows then
+ * keeps one tile of the device busy; the outputs are those of plh_forward either way.  Where it is 0 every
+ * row is computed (a caller that looks first saves more there: one row runs a smaller launch).
+ */
+int plh_detects_uniform(int input_size, int hidden_size, int num_layers, int output_size, int batch, int seq_len);
+int plh_forward_detect(const void* packed_dev, int input_size, int hidden_size, int num_layers, int output_size,
+                       const void* x, int batch, int seq_len, void* out, void* workspace, int64_t workspace_bytes,
+                       void* stream);
+
+/*
  * Time-parallel input projection: out[m][n] = sum_{j < k} x[m][j] * w[n][j] for m < rows, n < cols,
  * fp16 operands and result, fp32 accumulation (MFMA), e.g. one layer's x_t W_ih^T for all T steps
  * of a batch at once (rows = T * batch).

@@ -390,10 +390,21 @@ int64_t plh_workspace_bytes(int input_size, int hidden_size, int num_layers, int
                                         p.wide_rows ? 16 : p.tile_rows).total;
 }
 
-int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num_layers, int output_size,
-                const void* x, int batch, int seq_len, const int32_t* lengths, const void* h0, const void* c0,
-                void* out, void* out_seq, void* h_n, void* c_n, const int32_t* probe_steps, int n_probe,
-                float* probe_h, float* probe_c, void* workspace, int64_t workspace_bytes, void* stream) {
+}  // extern "C"
+
+namespace {
+
+// True if the whole batch runs in one wavefront launch of 8-row tiles: what one row of it would run, so
+// detecting a batch of equal rows saves no launch, and the kernel can do it on the way.
+bool detects_uniform(const plh::Geometry& g, const Plan& plan, int batch) {
+  return !plan.rec && !plan.wide_rows && g.slices == 1 && plan.tile_rows == 8 && batch > 1 && batch <= plan.chunk_rows;
+}
+
+int forward_impl(const void* packed_dev, int input_size, int hidden_size, int num_layers, int output_size,
+                 const void* x, int batch, int seq_len, const int32_t* lengths, const void* h0, const void* c0,
+                 void* out, void* out_seq, void* h_n, void* c_n, const int32_t* probe_steps, int n_probe,
+                 float* probe_h, float* probe_c, void* workspace, int64_t workspace_bytes, void* stream,
+                 bool detect) {
   plh::Geometry g;
   if (!geometry(input_size, hidden_size, num_layers, output_size, &g))
     return geometry_code(input_size, hidden_size, num_layers, output_size);
@@ -551,6 +562,12 @@ int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num
       a.gates = (const _Float16*)(ws + w.gates);
       a.wih_up = (const _Float16*)(pk + p.wih) + (size_t)4 * g.HP * g.kp0;
     }
+    if (detect && detects_uniform(g, plan, batch) && seq_len > 0) {
+      // The prologue blocks' verdicts go behind the status word, up to xp (the wavefront kernel uses no
+      // counters there): 127 words at least.
+      a.uniform = status + 1;
+      a.n_uniform = (int)std::min(w.xp / 4 - 1, (size_t)INT_MAX);
+    }
     err = plh::launch_forward_prologue(g, a, row0 == 0 ? status : nullptr, plan.wide_rows ? 0 : g.g_in0,
                                        w.xring_words, s);
     if (err != hipSuccess) return fail_hip(err, "forward prologue");
@@ -576,6 +593,35 @@ int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num
     ++tm.used;
   }
   return PLH_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int plh_forward(const void* packed_dev, int input_size, int hidden_size, int num_layers, int output_size,
+                const void* x, int batch, int seq_len, const int32_t* lengths, const void* h0, const void* c0,
+                void* out, void* out_seq, void* h_n, void* c_n, const int32_t* probe_steps, int n_probe,
+                float* probe_h, float* probe_c, void* workspace, int64_t workspace_bytes, void* stream) {
+  return forward_impl(packed_dev, input_size, hidden_size, num_layers, output_size, x, batch, seq_len, lengths, h0, c0,
+                      out, out_seq, h_n, c_n, probe_steps, n_probe, probe_h, probe_c, workspace, workspace_bytes,
+                      stream, false);
+}
+
+int plh_detects_uniform(int input_size, int hidden_size, int num_layers, int output_size, int batch, int seq_len) {
+  plh::Geometry g;
+  if (!geometry(input_size, hidden_size, num_layers, output_size, &g) || batch < 0 || seq_len < 0) return 0;
+  hipError_t err = hipSuccess;
+  const Plan plan = plan_for(g, batch, seq_len, true, &err);
+  return err == hipSuccess && detects_uniform(g, plan, batch) ? 1 : 0;
+}
+
+int plh_forward_detect(const void* packed_dev, int input_size, int hidden_size, int num_layers, int output_size,
+                       const void* x, int batch, int seq_len, void* out, void* workspace, int64_t workspace_bytes,
+                       void* stream) {
+  return forward_impl(packed_dev, input_size, hidden_size, num_layers, output_size, x, batch, seq_len, nullptr, nullptr,
+                      nullptr, out, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, workspace,
+                      workspace_bytes, stream, true);
 }
 
 int plh_forward_noalloc(const void* packed_dev, int input_size, int hidden_size, int num_layers, int output_size,

@@ -147,6 +147,10 @@ struct ForwardArgs {
                                 // wg_tiles, rounded up to 8 the same way; 0: exactly those)
   const _Float16* gates;        // [T * rows_pad][4 HP] blocked: input projection of that layer (no bias), lane order
                                 // (wavefront kernel: of layer 0, where the input is wider than HP; else null)
+  uint32_t* uniform;            // uniform-batch detection: one word per prologue block, nonzero if it saw a row that
+                                // differs from row 0 (null: no detection).  The wavefront kernel's 8-row tiles of a
+                                // batch in one launch only
+  int n_uniform;
   const _Float16* wih_up;       // wavefront kernel with gates: W_ih of layers 1.., [4 HP][HP] each, rows in lane order
   _Float16* hout;               // [T * rows_pad][HP] blocked: its h sequence, the next layer's input (null: last layer)
   const _Float16* wx0;          // rec_x0, layer 0: W_ih fragments of the in-kernel projection (x from xp)
@@ -161,7 +165,9 @@ hipError_t launch_pack_linear(const Geometry& g, const _Float16* w, const _Float
 // One launch before each persistent launch: packs this launch's x into xp (g0 8-wide K groups per
 // row and step, zero past I) and clears the status word (if `status`), the counters and ring_words
 // u64 words (an even number) of the exchange ring, or for the wavefront kernels their hand-off rings.
-hipError_t launch_forward_prologue(const Geometry& g, const ForwardArgs& a, uint32_t* status, int g0,
+// With a.uniform (a.n_uniform words of it) it also compares every row with row 0, and sets a.n_uniform to the
+// words it fills.
+hipError_t launch_forward_prologue(const Geometry& g, ForwardArgs& a, uint32_t* status, int g0,
                                    size_t ring_words, hipStream_t s);
 hipError_t launch_zero_u32(uint32_t* p, size_t n, hipStream_t s);
 hipError_t launch_repeat_first_row(const _Float16* in, _Float16* out, int rows, int cols, hipStream_t s);

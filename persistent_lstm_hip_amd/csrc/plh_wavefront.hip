@@ -147,6 +147,16 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
     Tt = __builtin_amdgcn_readfirstlane(lds.tlen);  // steps this tile runs: the longest row in it
   }
 
+  // A batch of equal rows (seen by the prologue's blocks): only the first tile runs, and its head writes
+  // row 0's outputs for every row.
+  bool uniform = false;
+  if (!RAGGED && a.uniform) {
+    uint32_t differs = 0;
+    for (int i = threadIdx.x; i < a.n_uniform; i += NT) differs |= a.uniform[i];
+    uniform = __syncthreads_or(differs != 0u) == 0;
+    if (uniform && tile != 0) return;
+  }
+
   // Resident weights: A fragments of [W_ih | W_hh] rows for this wave's 16 units, 4 gates.
   f16x8 w[KC][4];
   if constexpr (!WIDE) {
@@ -648,7 +658,7 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
     // output of this workgroup (states, probes, output sequence, head) and leave.
     if (row_ok) poison_lane_outputs(a, layer, grow, uo, UPL, !DOWN);
     if (!DOWN && a.out) {
-      for (int idx = threadIdx.x; idx < ROWS * a.O; idx += NT) {
+      for (int idx = threadIdx.x; idx < (uniform ? a.B : ROWS) * a.O; idx += NT) {
         const int g = a.row0 + tile * ROWS + idx / a.O;
         if (g < a.row_end) a.out[(size_t)g * a.O + idx % a.O] = (_Float16)__builtin_nanf("");
       }
@@ -685,6 +695,8 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
   // Linear head on the final h of the last layer (slot of the tile's last step).
   if (!DOWN && a.out) {
     const _Float16* hf = reinterpret_cast<const _Float16*>(lds.hist[(Tt + 1) & 1]);
+    _Float16* const row0_out = reinterpret_cast<_Float16*>(lds.xin);  // (no step reads the inputs any more)
+    static_assert(sizeof(lds.xin) >= 4096 * sizeof(_Float16), "one row of the widest head");
     for (int idx = threadIdx.x; idx < ROWS * a.O; idx += NT) {
       const int rr = idx / a.O, o = idx % a.O;
       const int g = a.row0 + tile * ROWS + rr;
@@ -699,7 +711,13 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
           s1 = fmaf((float)hv[j + 1], wr[k8 + j + 1], s1);
         }
       }
-      a.out[(size_t)g * a.O + o] = (_Float16)(a.blin[o] + (s0 + s1));
+      const _Float16 y = (_Float16)(a.blin[o] + (s0 + s1));
+      a.out[(size_t)g * a.O + o] = y;
+      if (rr == 0) row0_out[o] = y;
+    }
+    if (uniform) {
+      __syncthreads();
+      for (int idx = ROWS * a.O + threadIdx.x; idx < a.B * a.O; idx += NT) a.out[idx] = row0_out[idx % a.O];
     }
   }
 }

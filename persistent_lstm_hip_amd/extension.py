@@ -54,6 +54,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.plh_forward.argtypes = (
         [_vp] + [_i32] * 4 + [_vp, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _vp, _i64, _vp]
     )
+    lib.plh_detects_uniform.restype = _i32
+    lib.plh_detects_uniform.argtypes = [_i32] * 6
+    lib.plh_forward_detect.restype = _i32
+    lib.plh_forward_detect.argtypes = [_vp] + [_i32] * 4 + [_vp, _i32, _i32, _vp, _vp, _i64, _vp]
     lib.plh_status.restype = _i32
     lib.plh_status.argtypes = [_vp, ctypes.POINTER(ctypes.c_uint32), _vp]
     lib.plh_kernel_timing.restype = _i32
@@ -332,6 +336,31 @@ class NativeLibrary:
         if P:
             res["probe_h"], res["probe_c"] = probe_h, probe_c
         return res
+
+    def detects_uniform(self, dims: Sequence[int], batch: int, seq_len: int, device: torch.device) -> bool:
+        """True if forward_detect finds a batch of equal rows on the device at no cost to other batches."""
+        with _on_device(device):
+            return bool(self.lib.plh_detects_uniform(*dims, batch, seq_len))
+
+    def forward_detect(self, packed: torch.Tensor, dims: Sequence[int], x: torch.Tensor) -> torch.Tensor:
+        """plh_forward_detect: the head outputs [B, O] of full-length rows x [B, T, I] on a HIP device."""
+        I, H, L, O = dims
+        device = x.device
+        if int(x.size(2)) != I:
+            raise ValueError(f"x has input size {int(x.size(2))}, the model expects {I}")
+        if not x.is_floating_point():
+            raise ValueError("x must be a floating-point tensor")
+        if packed.device != device:
+            raise ValueError("packed weights and x must be on the same device")
+        B, T = int(x.size(0)), int(x.size(1))
+        xh = (x if x.dtype is torch.float16 else x.to(torch.float16)).contiguous()
+        out = torch.empty((B, O), device=device, dtype=torch.float16)
+        with _on_device(device):
+            ws = self.workspace(device, self.workspace_bytes(I, H, L, O, B, T))
+            rc = self.lib.plh_forward_detect(packed.data_ptr(), I, H, L, O, xh.data_ptr(), B, T, out.data_ptr(),
+                                             ws.data_ptr(), ws.numel(), _stream(device))
+        self._check(rc, "plh_forward_detect")
+        return out
 
     def status(self, device: torch.device) -> int:
         """Synchronise the current stream and return the device status word of the last forward."""

@@ -297,12 +297,18 @@ class PersistentLSTMRegressor(nn.Module):
         blob = self.lstm.packed_blob(x.device, self.linear)
         dims = self.dims()
         batch = int(x.size(0))
-        uniform = self._should_use_uniform_batch_fast_path(x)
+        # In auto mode a batch that runs in one launch of the same kernel as one of its rows is compared on
+        # the device, by the launch that packs x: no host synchronisation in front of the forward.
+        on_device = batch > 1 and _uniform_mode() in _AUTO and ext.detects_uniform(dims, batch, int(x.size(1)), x.device)
+        uniform = False if on_device else self._should_use_uniform_batch_fast_path(x)
         if not self._debug_reported and _debug():
             print(f"persistent_lstm_hip_amd debug: backend={BACKEND_NAME}, batch={batch}, "
-                  f"seq_len={int(x.size(1))}, dims={dims}, uniform_batch_fast_path={uniform}")
+                  f"seq_len={int(x.size(1))}, dims={dims}, "
+                  f"uniform_batch_fast_path={'on device' if on_device else uniform}")
             self._debug_reported = True
-        if uniform:
+        if on_device:
+            out = ext.forward_detect(blob, dims, x)
+        elif uniform:
             row = ext.forward(blob, dims, x.narrow(0, 0, 1))["out"]
             out = ext.repeat_first_row(row, batch)
         else:

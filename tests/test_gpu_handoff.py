@@ -12,7 +12,7 @@ import torch
 
 from conftest import make_regressor, make_x, oracle_layers
 from oracle import oracle
-from persistent_lstm_hip_amd import PersistentLSTM
+from persistent_lstm_hip_amd import PersistentLSTM, PersistentLSTMRegressor
 
 pytestmark = pytest.mark.gpu
 BOUND = 2e-3
@@ -106,3 +106,22 @@ def test_wide_inputs(gpu, I, H, L, B, T):
         want = _oracle(native, x[rows], lengths=None if lens is None else lens.numpy()[rows])
         assert np.abs(res["out_seq"].float().cpu().numpy()[rows] - want["out_seq"]).max() <= 2 * BOUND
         assert np.abs(res["h_n"].float().cpu().numpy()[:, rows] - want["h_n"]).max() <= 2 * BOUND
+
+
+@pytest.mark.parametrize("I,H,L,B,T", [(5, 128, 4, 512, 60), (1, 20, 1, 2, 1), (9, 64, 2, 33, 17), (128, 128, 2, 9, 40)])
+def test_equal_rows_found_on_the_device(gpu, monkeypatch, I, H, L, B, T):
+    """Equal rows, and equal but for one element (the last one, the first one of row 1, the middle of a row):
+    the outputs are bit for bit those of a forward without detection."""
+    print(f"[gpu-case] uniform I={I} H={H} L={L} B={B} T={T}", flush=True)
+    model = PersistentLSTMRegressor.from_native_module(make_regressor(I, H, L, 11)).to("cuda").half().eval()
+    assert gpu.detects_uniform((I, H, L, 11), B, T, torch.device("cuda"))
+    row = make_x(1, T, I, seed=2).to("cuda", torch.float16)
+    for where in (None, (B - 1, T - 1, I - 1), (1, 0, 0), (B // 2, T // 2, I // 2)):
+        x = row.expand(B, T, I).contiguous()
+        if where is not None and where[0] > 0:
+            x[where] += 1
+        monkeypatch.setenv("PERSISTENT_LSTM_HIP_UNIFORM_BATCH", "auto")
+        got = model(x)
+        gpu.check_status(torch.device("cuda"))
+        monkeypatch.setenv("PERSISTENT_LSTM_HIP_UNIFORM_BATCH", "0")
+        assert torch.equal(got, model(x)), where
