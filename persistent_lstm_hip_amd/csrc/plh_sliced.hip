@@ -34,10 +34,15 @@
 // Reference behaviour restated (mantuoluozk/persistent_lstm_hip): the generic path's recurrence
 // (persistent_lstm_hip.cu:2923-3181) with the input projection kept in fp32, gate order i, f, g, o
 // and the c/h recurrence of persistent_lstm_reference.cpp:21-35.
+#include <type_traits>
+
 #include "plh_device.h"
 
 namespace plh {
 namespace {
+
+template <int K>
+using Chunk = std::integral_constant<int, K>;
 
 template <int HP, int NTI>
 __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
@@ -284,14 +289,23 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
   auto clamp_step = [&](int s) { return s < Tt ? s : Tt - 1; };
 
   // ---- MFMA parts of a step ----
+  // K chunk of a tile's input part in front of which the polls of its exchange are issued: the MFMAs behind
+  // cover the polls' round trip, those in front the time the siblings' words need to arrive (a poll that
+  // finds one missing costs a round trip more).  Interleaved runs on one box, polls after all of the input
+  // part (one tile) or in front of it (two) -> here: H512 B64 2.02 -> 1.92 us per step, H400 L2 B40 1.90 ->
+  // 1.80, H256 B64 1.54 -> 1.47, L1 B8 1.35 -> 1.29, C3 (two tiles) 2.69 -> 2.63.  For one tile 1/4 and 3/4 were
+  // slower at H 256, 1/4 and 0 at H 512 (up to +10%); for two tiles 1/8 and 1/2.
+  constexpr int kPollChunk = NTI == 2 ? KCH / 4 : HP == 512 ? KCH * 3 / 4 : KCH / 2;
   f32x4 acc[NTI][NJ];
-  // acc[i] = bias + x_s W_ih^T of tile i (x_s in ring slot s & 1).
-  auto input_mfma = [&](int i, int s) {
+  // acc[i] = bias + x_s W_ih^T of tile i (x_s in ring slot s & 1), K chunks k0 .. k1 - 1 of it.
+  auto input_mfma = [&](int i, int s, auto k0, auto k1) {
+    constexpr int K0 = decltype(k0)::value, K1 = decltype(k1)::value;
     const f16x8* src = ring[i][s & 1] + lane;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = f32x4{bias[0][j], bias[1][j], bias[2][j], bias[3][j]};
+    for (int j = 0; j < NJ; ++j)
+      if (K0 == 0) acc[i][j] = f32x4{bias[0][j], bias[1][j], bias[2][j], bias[3][j]};
 #pragma unroll
-    for (int kc = 0; kc < KCH; ++kc) {
+    for (int kc = K0; kc < K1; ++kc) {
       const f16x8 bv = src[kc * FV];
 #pragma unroll
       for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[kc][j], bv, acc[i][j], 0, 0, 0);
@@ -400,10 +414,9 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
     else
       __builtin_amdgcn_raw_buffer_store_b64(wd, slot_rs(i, t), woff, 0, 16);
   };
-  // The polls of tile i's step t, issued after the tile's word and (two tiles) the other tile's cell
-  // update, when the siblings' words are usually written: a poll that finds a stale word costs a
-  // round trip at the gather.  Loads and stores retire in issue order, so the gather's wait covers
-  // nothing issued after these loads.
+  // The polls of tile i's step t, issued inside the tile's input part (kPollChunk), when the siblings' words
+  // are usually written.  Loads and stores retire in issue order, so the gather's wait covers nothing
+  // issued after these loads.
   auto issue_poll = [&](int i, int t) {
 #pragma unroll
     for (int p = 0; p < NLD; ++p) poll(i, t, p);
@@ -518,16 +531,15 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
   ok = __builtin_amdgcn_readfirstlane(s_fail) == 0;
   if (ok && Tt > 0) {
 #pragma unroll
-    for (int i = 0; i < NTI; ++i) input_mfma(i, 0);
+    for (int i = 0; i < NTI; ++i) input_mfma(i, 0, Chunk<0>(), Chunk<KCH>());
   }
   lds_barrier();  // step 0 overwrites ring slot 0 (with x_2) once every wave has read x_0
 
   // ---- steps ----
   // Step t, for both tiles of a two-tile workgroup at once (the exchange's round trip, the memory
   // issue and the barrier are paid once per step, not per tile): h_{t-1} W_hh^T; each tile's cell
-  // update, output sequence and word; the polls of step t, each followed by one tile's input part
-  // x_{t+1} W_ih^T, which covers the round trip (a poll issued right after the tile's own word would
-  // often find the siblings' words not yet written); the gathers into the other h buffer; then,
+  // update, output sequence and word; each tile's input part x_{t+1} W_ih^T (the last step computes a
+  // discarded one) with the polls of step t inside it; the gathers into the other h buffer; then,
   // off the step's chain, the input of step t + 2 into the ring, the hand-off copy of h_{t-1}, the
   // input pieces of step t + 3 and the counter (issued after the gathers, so that no wait of this
   // step covers them); one barrier, after which thread 0 publishes.
@@ -542,9 +554,11 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < NTI; ++i) {
-      if constexpr (NTI == 2) issue_poll(i, t);
-      if (t + 1 < Tt) input_mfma(i, t + 1);
-      if constexpr (NTI == 1) issue_poll(i, t);
+      input_mfma(i, t + 1, Chunk<0>(), Chunk<kPollChunk>());
+      __builtin_amdgcn_sched_barrier(0);
+      issue_poll(i, t);
+      __builtin_amdgcn_sched_barrier(0);
+      input_mfma(i, t + 1, Chunk<kPollChunk>(), Chunk<KCH>());
     }
 #pragma unroll
     for (int i = 0; i < NTI; ++i) gather(i, t, hbuf[i][(t + 1) & 1]);
