@@ -157,6 +157,12 @@ Plan plan_for(const plh::Geometry& g, int batch, int seq_len, bool need_device, 
   return n_wave > g.L ? q : p;
 }
 
+// The workspace layout a plan runs in.
+plh::WorkspaceLayout plan_layout(const plh::Geometry& g, const Plan& p, int seq_len) {
+  if (p.wide_rows) return plh::workspace_layout(plh::as_layer_sequential(g), seq_len, p.wide_rows, 16);
+  return plh::workspace_layout(p.rec ? plh::as_layer_sequential(g) : g, seq_len, p.chunk_rows, p.tile_rows);
+}
+
 bool geometry(int I, int H, int L, int O, plh::Geometry* g) {
   std::string why;
   if (!plh::make_geometry(I, H, L, O, g, &why)) {
@@ -385,9 +391,7 @@ int64_t plh_workspace_bytes(int input_size, int hidden_size, int num_layers, int
   }
   hipError_t err = hipSuccess;
   const Plan p = plan_for(g, batch, seq_len, false, &err);
-  if (p.rec || p.wide_rows) g = plh::as_layer_sequential(g);
-  return (int64_t)plh::workspace_layout(g, seq_len, p.wide_rows ? p.wide_rows : p.chunk_rows,
-                                        p.wide_rows ? 16 : p.tile_rows).total;
+  return (int64_t)plan_layout(g, p, seq_len).total;
 }
 
 }  // extern "C"
@@ -418,26 +422,24 @@ int forward_impl(const void* packed_dev, int input_size, int hidden_size, int nu
   hipStream_t s = (hipStream_t)stream;
 
   hipError_t err = hipSuccess;
-  const Plan plan = plan_for(g, batch, seq_len, true, &err);
+  const plh::Geometry base = g;
+  Plan plan = plan_for(base, batch, seq_len, true, &err);
   if (err != hipSuccess) return fail_hip(err, "occupancy query");
-  if (plan.rec) g = plh::as_layer_sequential(g);
+  if (plan.rec) g = plh::as_layer_sequential(base);
   const int tile_wgs = g.rec ? g.slices : g.L * g.slices;
   if (capacity(g, 16, &err) < tile_wgs)
     return fail(PLH_ERR_UNSUPPORTED, "the device cannot hold the " + std::to_string(tile_wgs) +
                                          " workgroups of one batch tile co-resident (layers = " +
                                          std::to_string(g.L) + ")");
-  const int chunk_rows = plan.chunk_rows;
-  const plh::WorkspaceLayout w =
-      plan.wide_rows ? plh::workspace_layout(plh::as_layer_sequential(g), seq_len, plan.wide_rows, 16)
-                     : plh::workspace_layout(g, seq_len, chunk_rows, plan.tile_rows);
-  if (workspace_bytes < (int64_t)w.total)
+  plh::WorkspaceLayout w = plan_layout(base, plan, seq_len);
+  const size_t ws_total = w.total;
+  if (workspace_bytes < (int64_t)ws_total)
     return fail(PLH_ERR_INVALID, "workspace smaller than plh_workspace_bytes()");
 
   const plh::PackedLayout p = plh::packed_layout(g);
   char* ws = (char*)workspace;
   const char* pk = (const char*)packed_dev;
   uint32_t* status = (uint32_t*)(ws + w.status);
-  uint32_t* counters = (uint32_t*)(ws + w.counters);
 
   StreamOrder order(s);
   if (order.error() != hipSuccess) return fail_hip(order.error(), "ordering against other streams' forwards");
@@ -450,14 +452,9 @@ int forward_impl(const void* packed_dev, int input_size, int hidden_size, int nu
   std::memset(&a, 0, sizeof(a));
   a.x = (const _Float16*)x;
   a.lengths = lengths;
-  a.wpack = (const _Float16*)(pk + (g.rec ? p.wrec : p.wpack));
   a.bias = (const float*)(pk + p.bias);
   a.wlin = (const float*)(pk + p.wlin);
   a.blin = (const float*)(pk + p.blin);
-  a.xp = (plh::f16x8_t*)(ws + w.xp);
-  a.hseq = (plh::f16x8_t*)(ws + w.hseq);
-  a.xring = (uint64_t*)(ws + w.xring);
-  a.counters = counters;
   a.status = status;
   a.h0 = (const _Float16*)h0;
   a.c0 = (const _Float16*)c0;
@@ -475,16 +472,35 @@ int forward_impl(const void* packed_dev, int input_size, int hidden_size, int nu
   a.H = g.H;
   a.L = g.L;
   a.O = g.O;
-  a.g_in0 = g.g_in0;
   a.wait_ticks = (uint64_t)g_wait_us * 100u;  // s_memrealtime: 100 MHz
   a.fail_step = g_fail_step;
 
   KernelTiming& tm = timing();
   const bool timed = tm.used * 2 < (int)tm.ev.size();
-  const int cus = g.rec || plan.wide_rows ? device_cus(&err) : 0;
+  const int cus = device_cus(&err);
   if (err != hipSuccess) return fail_hip(err, "device query");
-  for (int row0 = 0; row0 < batch; row0 += chunk_rows) {
-    const int rows = std::min(chunk_rows, batch - row0);
+  for (int row0 = 0; row0 < batch; row0 = a.row_end) {
+    if (row0 > 0 && batch - row0 < plan.chunk_rows) {
+      // The rows after the last full launch take the plan of a batch of their size, within the workspace
+      // laid out for the whole: 8-row tiles, one tile per workgroup, or the sliced path instead of the
+      // layer-sequential one (kernels of H128 L4 B1500 T250, 1024 + 476 rows: 617 -> 514 us; four layers of
+      // 500 steps at H256 B700 2.75 -> 2.08 ms, at H512 B600 8.69 -> 7.17 ms).
+      const Plan rest = plan_for(base, batch - row0, seq_len, true, &err);
+      if (err != hipSuccess) return fail_hip(err, "occupancy query");
+      const plh::WorkspaceLayout wr = plan_layout(base, rest, seq_len);
+      if (rest.fits && wr.total <= ws_total) {
+        plan = rest;
+        w = wr;
+        g = plan.rec ? plh::as_layer_sequential(base) : base;
+      }
+    }
+    a.wpack = (const _Float16*)(pk + (g.rec ? p.wrec : p.wpack));
+    a.xp = (plh::f16x8_t*)(ws + w.xp);
+    a.hseq = (plh::f16x8_t*)(ws + w.hseq);
+    a.xring = (uint64_t*)(ws + w.xring);
+    a.counters = (uint32_t*)(ws + w.counters);
+    a.g_in0 = g.g_in0;
+    const int rows = std::min(plan.chunk_rows, batch - row0);
     a.row0 = row0;
     a.row_end = row0 + rows;
     a.tile_rows = plan.tile_rows;
@@ -515,7 +531,7 @@ int forward_impl(const void* packed_dev, int input_size, int hidden_size, int nu
       // sequence, then the recurrent kernel, whose h sequence goes to the other xs slot.  The
       // exchange ring is cleared before each layer's launch (tags restart at 1).
       _Float16* xs[2] = {(_Float16*)(ws + w.xs),
-                         (_Float16*)(ws + w.xs) + (size_t)seq_len * chunk_rows * g.HP};
+                         (_Float16*)(ws + w.xs) + (size_t)seq_len * w.chunk_rows * g.HP};
       _Float16* gates = (_Float16*)(ws + w.gates);
       err = plh::launch_forward_prologue(g, a, row0 == 0 ? status : nullptr, g.rec_x0 ? 4 : 0, w.xring_words, s);
       if (err != hipSuccess) return fail_hip(err, "forward prologue");

@@ -125,3 +125,25 @@ def test_equal_rows_found_on_the_device(gpu, monkeypatch, I, H, L, B, T):
         gpu.check_status(torch.device("cuda"))
         monkeypatch.setenv("PERSISTENT_LSTM_HIP_UNIFORM_BATCH", "0")
         assert torch.equal(got, model(x)), where
+
+
+@pytest.mark.parametrize("I,H,L,B,T", [
+    (5, 128, 4, 1060, 40),    # 1024 rows in 16-row tiles, 36 in 8-row tiles
+    (5, 200, 4, 530, 12),     # two tiles per workgroup, then one
+    (5, 400, 4, 540, 12),     # layer by layer, then all layers at once
+    (300, 256, 2, 1030, 5),   # layer by layer twice
+    (5, 600, 2, 140, 6),      # padded H 1024: 128 rows, then 12
+])
+def test_rows_after_the_last_full_launch(gpu, I, H, L, B, T):
+    """A forward in several launches whose last one takes another plan: rows of both against the oracle
+    (layer-sequential rows also round their projections, as above), states and sequence included."""
+    print(f"[gpu-case] remainder I={I} H={H} L={L} B={B} T={T}", flush=True)
+    native = make_regressor(I, H, L, 3)
+    x = make_x(B, T, I, seed=8)
+    out, (h, c) = _lstm(native)(x.to("cuda", torch.float16))
+    gpu.check_status(torch.device("cuda"))
+    mid = 508 if B > 516 else 124
+    rows = np.unique(np.r_[0:4, mid:mid + 8, B - 12:B])
+    want = _oracle(native, x[rows])
+    assert np.abs(out.float().cpu().numpy()[rows] - want["out_seq"]).max() <= 2 * BOUND
+    assert np.abs(h.float().cpu().numpy()[:, rows] - want["h_n"]).max() <= 2 * BOUND
