@@ -197,8 +197,9 @@ proj_gemm_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* 
   }
 }
 
-// The blocked layouts at K = 32 KS (KS = 4, 8, 12 or 16: K = 128, 256, 384, 512), with the k-steps of an m-tile
-// unrolled at compile time.  The same work split, W slice and X ring as proj_gemm_kernel, written so
+// The blocked layouts: K = 32 KS (KS = 4, 8, 12 or 16: K = 128, 256, 384, 512), or MULTI: `blocks` K blocks of KS
+// k-steps each (K above 512: KS = 8, or 4 where K is an odd multiple of 128), with the k-steps of an m-tile
+// (MULTI: of a block) unrolled at compile time.  The same work split, W slice and X ring as proj_gemm_kernel, written so
 // that the compiler keeps the ring's loads kRing - 1 steps ahead everywhere: with a runtime k-loop the
 // register allocator rotated the ring slots through the accumulators and waited for every
 // outstanding load (vmcnt(0) / vmcnt(1)) twice per four k-steps.  Here
@@ -216,12 +217,19 @@ proj_gemm_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* 
 // [512000,512]x[512,2048] 1.03-1.05 -> 0.966-0.98 ms, [512000,128]x[128,512] 0.117 -> 0.109 ms
 // (interleaved runs on one box each); the stores in the next tile's first step: 0.943-0.951 ->
 // 0.933-0.935 ms and 0.105-0.106 -> 0.104-0.106 ms, bit-identical.
-template <int KS>
+//
+// MULTI: the W slice does not fit the LDS, so it is held one K block at a time, and the tiles take their blocks in
+// alternating order (up, down, up, ..): the block left by one tile is the next one's first, so a tile reloads
+// blocks - 1 of them, moved from global memory to LDS directly (16 bytes per lane, no registers).  Against the
+// run-time-K kernel, which reloads blocks of 512 twice per tile: [128000,1024]x[1024,4096] 1.10-1.16 -> 0.97-1.01
+// ms, K = 768 0.84-0.86 -> 0.71 ms, K = 640 0.73 -> 0.64 ms.  Blocks of 512 (the largest that fit) spilled 21 VGPRs
+// (+3%); two buffers, the next block loading under the current one's MFMAs, were 2-6% slower.
+template <int KS, bool MULTI>
 __global__ void __launch_bounds__(kGemmThreads)
-proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* __restrict__ W,
+proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* __restrict__ W, int blocks,
                          _Float16* __restrict__ C, long long ldc, int M, int tiles_m, int n_slices, int m_groups) {
   static_assert(kGemmWaves == 8 && kGemmWM == 4 && KS % kRing == 0 && KS * 32 <= kGemmMaxK, "tile shape");
-  constexpr int K = 32 * KS;
+  const int K = MULTI ? 32 * KS * blocks : 32 * KS;
   __shared__ f16x8 wl[KS * 8 * 64];  // [k-chunk][n-tile 0..7][64 lanes] f16x8
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
@@ -229,12 +237,24 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
   const int mg = (idx / n_slices) * 8 + xcd;
   if (mg >= m_groups) return;
   const int n0 = ns * kGemmBN;
-  for (int e = threadIdx.x; e < KS * 8 * 64; e += kGemmThreads) {
-    const int l = e & 63, nt = (e >> 6) & 7, kc = e >> 9;
-    const int n = n0 + gemm_w_row(nt, l & 15);
-    wl[e] = *reinterpret_cast<const f16x8*>(W + (size_t)n * K + kc * 32 + (l >> 4) * 8);
-  }
+  // K block b of the W slice into LDS (the caller's barriers around it): wave w loads n-tile w of every k-chunk.
+  const _Float16* const wsrc = W + (size_t)(n0 + gemm_w_row(wave, lane & 15)) * K + (lane >> 4) * 8;
+  auto load_w = [&](int b) {
+    const _Float16* const src = wsrc + b * (KS * 32);
+#pragma unroll
+    for (int i = 0; i < KS; ++i) {
+      f16x8* const dst = wl + (i * 8 + wave) * 64;
+      if constexpr (!MULTI)
+        dst[lane] = *reinterpret_cast<const f16x8*>(src + i * 32);
+      else
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(uintptr_t)(src + i * 32),
+                                         (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+    }
+    if constexpr (MULTI) wait_vmem_all();
+  };
+  load_w(0);
   __syncthreads();
+  int kb = 0, dir = 1;  // the K block in LDS, and the order of this tile's blocks
   int mt = mg;
   if (mt >= tiles_m) return;
   const int nblk = M / 16;
@@ -262,25 +282,25 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
     const auto rs = xrs(mt);
 #pragma unroll
     for (int j = 0; j < kRing - 1; ++j) {
-      ld(rs, j, xr[j]);
+      ld(rs, j, xr[j]);  // (the first tile starts with block 0)
       __builtin_amdgcn_sched_barrier(0);
     }
   }
   f32x4 acc[kGemmWM][8];
-  // k-step s of the tile whose X rows rc describes (rn: the next tile's, for the ring's loads past
-  // this tile's last step).  Step 0 starts every accumulator from zero; with `out` (a fused step 0)
+  // k-step s of the K block in LDS of the tile whose X rows rc describes; the ring's loads past the block's
+  // last step are the first ones of block nb of rn's rows (the tile's other block, or the next tile).  The `first` block's step 0 starts every accumulator from zero; with `out` (a fused step 0)
   // each accumulator pair of the previous tile is converted and stored right before the step's
   // MFMAs overwrite it, so the epilogue's VALU work and stores run beside the next tile's first
   // MFMAs instead of stalling the matrix core.
-  auto kstep = [&](int s, __amdgpu_buffer_rsrc_t rc, __amdgpu_buffer_rsrc_t rn, const __amdgpu_buffer_rsrc_t* out)
-      __attribute__((always_inline)) {
+  auto kstep = [&](int s, __amdgpu_buffer_rsrc_t rc, __amdgpu_buffer_rsrc_t rn, int nb, bool first,
+                   const __amdgpu_buffer_rsrc_t* out) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
     {
       const int sn = s + kRing - 1;  // this tile's step sn, or the next tile's first steps
       if (sn < KS)
-        ld(rc, sn, xr[sn % kRing]);
+        ld(rc, kb * KS + sn, xr[sn % kRing]);
       else
-        ld(rn, sn - KS, xr[sn % kRing]);
+        ld(rn, nb * KS + sn - KS, xr[sn % kRing]);
     }
     f16x8 wa[3];
     wa[0] = wl[(s * 8 + 0) * 64 + lane];
@@ -306,7 +326,7 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
 #pragma unroll
       for (int a = 0; a < kGemmWM; ++a)
         acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wa[b % 3], xr[s % kRing][a],
-                                                          s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[a][b], 0, 0, 0);
+                                                          first && s == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[a][b], 0, 0, 0);
     }
     // issue order (masks: 0x020 vector-memory reads, 0x100 LDS reads, 0x008 MFMA, 0x002 VALU,
     // 0x040 vector-memory writes)
@@ -351,9 +371,29 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
     const int nmt = mt + m_groups;
     const int pmt = nmt < tiles_m ? nmt : mt;  // prefetch target past the last tile: reload this one
     const auto rc = xrs(mt), rn = xrs(pmt);
-    kstep(0, rc, rn, &prev);
+    if constexpr (!MULTI) {
+      kstep(0, rc, rn, 0, true, &prev);
 #pragma unroll
-    for (int s = 1; s < KS; ++s) kstep(s, rc, rn, nullptr);
+      for (int s = 1; s < KS; ++s) kstep(s, rc, rn, 0, true, nullptr);
+    } else {
+      kstep(0, rc, rc, kb + dir, true, &prev);
+#pragma unroll
+      for (int s = 1; s < KS; ++s) kstep(s, rc, rc, kb + dir, true, nullptr);
+#pragma unroll 1
+      for (int j = 1; j < blocks; ++j) {
+        // every wave is done with the block (its MFMAs read it from registers loaded before them)
+        __syncthreads();
+        kb += dir;
+        load_w(kb);
+        __syncthreads();
+        const bool more = j + 1 < blocks;
+        const auto rx = more ? rc : rn;
+        const int nb = more ? kb + dir : kb;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) kstep(s, rc, rx, nb, false, nullptr);
+      }
+      dir = -dir;
+    }
     __builtin_amdgcn_sched_barrier(0);
     prev = crs(mt);
     if (nmt >= tiles_m) break;
@@ -392,14 +432,16 @@ hipError_t launch_proj_gemm(const _Float16* X, long long ldx, const _Float16* W,
   const int m_groups = std::max(1, std::min(tiles_m, std::max(cus, 1) / n_slices));
   const int grid = ((m_groups + 7) / 8) * 8 * n_slices;
   // The compile-time-K kernel where one is built (other K: the generic kernel).
+  const bool multi = K > kGemmMaxK;
   auto* fk = !blocked || ldc > (1 << 20) ? nullptr
-             : K == 128                   ? proj_gemm_blocked_kernel<4>
-             : K == 256                   ? proj_gemm_blocked_kernel<8>
-             : K == 384                   ? proj_gemm_blocked_kernel<12>
-             : K == 512                   ? proj_gemm_blocked_kernel<16>
-                                          : nullptr;
+             : multi                      ? (K % 256 == 0 ? proj_gemm_blocked_kernel<8, true> : proj_gemm_blocked_kernel<4, true>)
+             : K == 128                   ? proj_gemm_blocked_kernel<4, false>
+             : K == 256                   ? proj_gemm_blocked_kernel<8, false>
+             : K == 384                   ? proj_gemm_blocked_kernel<12, false>
+                                          : proj_gemm_blocked_kernel<16, false>;
   if (fk) {
-    hipLaunchKernelGGL(fk, dim3(grid), dim3(kGemmThreads), 0, s, X, ldx, W, C, ldc, (int)M, tiles_m, n_slices, m_groups);
+    hipLaunchKernelGGL(fk, dim3(grid), dim3(kGemmThreads), 0, s, X, ldx, W, multi ? K / (K % 256 == 0 ? 256 : 128) : 1, C,
+                       ldc, (int)M, tiles_m, n_slices, m_groups);
     return hipGetLastError();
   }
   const bool kb = K > kGemmMaxK;

@@ -91,3 +91,17 @@ def test_input_projection_rejects_bad_shapes(gpu):
     for xs, ws in (((10, 96), (256, 96)), ((10, 128), (200, 128)), ((10, 650), (256, 650))):
         with pytest.raises(ValueError, match="k % 128"):
             gpu.input_projection(z(*xs), z(*ws))
+
+
+@pytest.mark.parametrize("rows,k,cols", [(16, 640, 128), (528, 768, 256), (8208, 896, 128), (1040, 1024, 384), (32, 2176, 128)])
+def test_blocked_gemm_k_blocks(gpu, rows, k, cols):
+    """K above 512 in blocks of 256 or 128, taken in alternating order by successive row tiles: one tile, a
+    tile and a remainder, several tiles per workgroup; an odd and an even number of blocks.  fp16 results of
+    fp32 sums: half an ulp (2^-11 of the value) plus the sums' own rounding."""
+    print(f"[gpu-case] blocked GEMM rows={rows} k={k} cols={cols}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = torch.randn(rows, k, device="cuda", generator=g).half()
+    w = (torch.randn(cols, k, device="cuda", generator=g) / k ** 0.5).half()
+    got = gpu.from_blocked(gpu.input_projection(gpu.to_blocked(x), w, blocked=True)).double()
+    want = x.double() @ w.double().t()
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + 1e-4).all()
