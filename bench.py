@@ -388,7 +388,7 @@ def main() -> int:
         "latency_s": median_ms * 1e-3,
         "latency_100_fwd_wall_s": wall * 100.0 / args.steps,
         "kernel": {
-            "name": "lstm_wavefront_kernel<128,8,8,false>",
+            "name": "lstm_wavefront_kernel<128,8,false,false>",
             "avg_ms": kernel_ms,
             "per_step_us": kernel_ms * 1e3 / (T + L - 1),
             "timed_launches": n_timed,

@@ -96,13 +96,16 @@ int64_t plh_workspace_bytes(int input_size, int hidden_size, int num_layers, int
  * device are ordered by the library (each needs the whole device co-resident): the first forward
  * on a second stream synchronises the device once, later ones wait on an event of the previous
  * forward when it was on another stream (not inside a stream capture).  Hidden sizes 513..1024, inputs wider
- * than the padded hidden size, and at padded H 512 a batch that needs more wavefront launches than
+ * than the padded hidden size above 128, and at padded H 512 a batch that needs more wavefront launches than
  * there are layers run layer by layer: per layer the input projection of every step as one fp16
  * MFMA GEMM (plh_input_projection's kernel; for layer 0 with input_size <= 32 at H > 256 inside the
  * recurrent kernel), then a W_hh-only persistent kernel.  That path rounds the GEMM's x_t W_ih^T to
  * fp16 before the recurrent sum, as the reference's generic path does (persistent_lstm_hip.cu:
  * 2988-2994); the all-layers path keeps it in fp32, so at padded H 512 the batch size decides which
- * of the two roundings a row gets (both are within the tolerance).
+ * of the two roundings a row gets (both are within the tolerance; the rows after the last full launch of
+ * a batch take the path of a batch of their number).  At padded H 128 an input wider than that has its
+ * layer-0 projections from the same GEMM, rounded to fp16, in front of one launch of all layers (short
+ * sequences of more than three layers: layer by layer).
  * Replaces persistent_lstm4_forward_interleaved (bindings.cpp:157, persistent_lstm_hip.cu:2126-2254)
  * and persistent_lstm_regressor_forward_generic_projected (bindings.cpp:163,
  * persistent_lstm_hip.cu:2923-3181), whose signatures return only the [batch, O] head output;

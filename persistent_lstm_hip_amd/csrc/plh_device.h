@@ -55,27 +55,6 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Spin (one lane) until *ctr >= need, bounded by `limit` ticks of s_memrealtime (100 MHz), then
-// acquire at agent scope.  Returns 0 if the wait timed out or any workgroup of the grid has failed.
-__device__ __attribute__((unused)) int wait_counter(const uint32_t* ctr, uint32_t need, uint32_t* status, uint64_t limit) {
-  uint32_t v = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (v < need) {
-    const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-    for (;;) {
-      __builtin_amdgcn_s_sleep(1);
-      v = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (v >= need) break;
-      if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return 0;
-      if (__builtin_amdgcn_s_memrealtime() - t0 > limit) {
-        __hip_atomic_fetch_or(status, PLH_STATUS_TIMEOUT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return 0;
-      }
-    }
-  }
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-  return __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u ? 1 : 0;
-}
-
 // After a failed wait: NaN into every output element a lane owns, units u0 + stride * j (j < n) of
 // batch row `grow` in `layer`: h_n, c_n, every probe and, for the last layer, every step of out_seq.
 // With the head poisoned as well, each output element of a forward is then either its correct value

@@ -10,16 +10,15 @@
 //     the B columns 8..15 repeat rows 0..7 and each lane evaluates two of its four (unit, row)
 //     pairs; the next step's input part is issued between this step's gate computations;
 //   * the gate nonlinearities and the c/h update run on the accumulator registers; c never leaves
-//     VGPRs; h goes to an LDS history (double-buffered by chunk) that also feeds the next step's
-//     recurrent MFMAs and the hand-off copy;
+//     VGPRs; h goes to LDS (double-buffered by step) for the next step's recurrent MFMAs;
 //   * activations live in "fragment order": a [R rows x 32 k] block is stored as [k/8][row][8],
-//     i.e. exactly the B operand of one MFMA (lane l reads 16 B at l * 16), in LDS and in the
-//     global hand-off buffer, so LDS traffic is conflict-free and global traffic contiguous;
+//     i.e. exactly the B operand of one MFMA (lane l reads 16 B at l * 16), so LDS traffic is
+//     conflict-free;
 //   * a layer hands h to the next one step by step: each lane sends its units of h_t as one tagged word
 //     through a ring of kHandoffSlots steps per (layer, tile), and the same lane of the next layer's
 //     workgroup loads it four steps ahead, checks its tag two steps ahead and puts it into LDS.  No
 //     counter, barrier or fence sits between the two layers, so layer l+1 runs about six steps behind
-//     layer l (measured: C1-sized T = 64, L = 4, B = 1 87 -> 57 us against chunks of 8 steps, which lagged 18
+//     layer l (measured: the kernel of H 128, L = 4, B = 1, T = 64 87 -> 62 us against chunks of 8 steps, which lagged 18
 //     steps per layer; C2 853 -> 787 us, where a chunk's copies also cost ~10% of the steps).  The sends,
 //     loads and checks sit under the latency of the step's LDS reads of h.  Where the ring wraps,
 //     counters read once per 8 steps keep a layer from running a whole ring ahead;

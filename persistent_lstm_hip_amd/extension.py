@@ -13,6 +13,7 @@ against `persistent_lstm_hip_ext` keeps working.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from functools import lru_cache
@@ -104,22 +105,25 @@ def _device_key(device: torch.device) -> tuple:
     return (device.type, index, torch._C._cuda_getCurrentRawStream(index))
 
 
-class _on_device:
-    """torch.cuda.device(device) that does nothing when it is already the current device."""
+_CURRENT = contextlib.nullcontext()
 
-    __slots__ = ("index", "prev")
 
-    def __init__(self, device: torch.device):
-        self.index = _index(device)
+def _on_device(device: torch.device):
+    """torch.cuda.device(device), or nothing when it is already the current device."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return _CURRENT
+    return torch.cuda.device(device.index)
 
-    def __enter__(self) -> None:
-        self.prev = torch.cuda.current_device()
-        if self.prev != self.index:
-            torch.cuda.set_device(self.index)
 
-    def __exit__(self, *exc) -> None:
-        if self.prev != self.index:
-            torch.cuda.set_device(self.prev)
+def _launch(device: torch.device, fn, *args) -> int:
+    """fn(*args, the device's current stream) with the device current."""
+    current = torch.cuda.current_device()
+    index = current if device.index is None else device.index
+    stream = torch._C._cuda_getCurrentRawStream(index)
+    if index == current:
+        return fn(*args, stream)
+    with torch.cuda.device(index):
+        return fn(*args, stream)
 
 
 class NativeLibrary:
@@ -206,11 +210,8 @@ class NativeLibrary:
         lw, lb = half(lin_w), half(lin_b)
         nbytes = self.packed_bytes(I, H, L, O)
         packed = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        with _on_device(device):
-            rc = self.lib.plh_pack_regressor(
-                I, H, L, O, a_wih, a_whh, a_bih, a_bhh, _ptr(lw), _ptr(lb), packed.data_ptr(), nbytes,
-                _stream(device),
-            )
+        rc = _launch(device, self.lib.plh_pack_regressor, I, H, L, O, a_wih, a_whh, a_bih, a_bhh, _ptr(lw), _ptr(lb),
+                     packed.data_ptr(), nbytes)
         self._check(rc, "plh_pack_regressor")
         # The fp16 copies in `keep` are read asynchronously; the caching allocator only hands their
         # blocks to later work on the same stream, which runs after the pack kernels.
@@ -364,12 +365,12 @@ class NativeLibrary:
 
     def status(self, device: torch.device) -> int:
         """Synchronise the current stream and return the device status word of the last forward."""
+        device = torch.device(device)
         ws = self._workspaces.get(_device_key(device))
         if ws is None:
             return 0
         st = ctypes.c_uint32(0)
-        with _on_device(device):
-            self._check(self.lib.plh_status(ws.data_ptr(), ctypes.byref(st), _stream(device)), "plh_status")
+        self._check(_launch(device, self.lib.plh_status, ws.data_ptr(), ctypes.byref(st)), "plh_status")
         return int(st.value)
 
     def check_status(self, device: torch.device) -> None:
@@ -442,9 +443,8 @@ class NativeLibrary:
               or (blocked and not out.is_contiguous())):
             raise ValueError("out must be a float16 [rows, cols] tensor with unit column stride (blocked: contiguous)")
         ldo = cols if (blocked or rows <= 1) else int(out.stride(0))
-        with _on_device(x.device):
-            rc = self.lib.plh_input_projection(x.data_ptr(), ldx, w.data_ptr(), k, out.data_ptr(), ldo, rows, cols,
-                                               1 if blocked else 0, _stream(x.device))
+        rc = _launch(x.device, self.lib.plh_input_projection, x.data_ptr(), ldx, w.data_ptr(), k, out.data_ptr(), ldo,
+                     rows, cols, 1 if blocked else 0)
         self._check(rc, "plh_input_projection")
         return out
 
@@ -471,9 +471,8 @@ class NativeLibrary:
         inp = inp.contiguous()
         cols = int(inp.size(1))
         out = torch.empty((int(output_batch_size), cols), dtype=inp.dtype, device=inp.device)
-        with _on_device(inp.device):
-            rc = self.lib.plh_repeat_first_row(inp.data_ptr(), out.data_ptr(), int(output_batch_size), cols,
-                                               _stream(inp.device))
+        rc = _launch(inp.device, self.lib.plh_repeat_first_row, inp.data_ptr(), out.data_ptr(), int(output_batch_size),
+                     cols)
         self._check(rc, "plh_repeat_first_row")
         return out
 

@@ -41,9 +41,10 @@ def test_lengths_around_the_ring(gpu, H, L, B, T):
     assert np.abs(c.float().cpu().numpy() - want["c_n"]).max() <= 2 * BOUND
 
 
-@pytest.mark.parametrize("H,L,B,T", [(128, 2, 1100, 41), (60, 4, 40, 70)])
+@pytest.mark.parametrize("H,L,B,T", [(128, 2, 1100, 41), (60, 4, 40, 70), (128, 5, 400, 70)])
 def test_ragged_rows_and_tiles(gpu, H, L, B, T):
-    """16-row tiles (1100 rows) and 8-row tiles; lengths 0 .. T, rows of length 0 with |h0| up to 3."""
+    """16-row tiles (1100 rows) and 8-row tiles, of five layers on different XCDs too (50 tiles, which the grid
+    has no room to round up); lengths 0 .. T, rows of length 0 with |h0| up to 3."""
     print(f"[gpu-case] hand-off ragged H={H} L={L} B={B} T={T}", flush=True)
     native = make_regressor(5, H, L, 3)
     x = make_x(B, T, 5, seed=3)
