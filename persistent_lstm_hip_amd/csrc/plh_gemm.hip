@@ -288,10 +288,11 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
   }
   f32x4 acc[kGemmWM][8];
   // k-step s of the K block in LDS of the tile whose X rows rc describes; the ring's loads past the block's
-  // last step are the first ones of block nb of rn's rows (the tile's other block, or the next tile).  The `first` block's step 0 starts every accumulator from zero; with `out` (a fused step 0)
-  // each accumulator pair of the previous tile is converted and stored right before the step's
-  // MFMAs overwrite it, so the epilogue's VALU work and stores run beside the next tile's first
-  // MFMAs instead of stalling the matrix core.
+  // last step are the first ones of block nb of rn's rows (the tile's other block, or the next tile).  The
+  // `first` block's step 0 starts every accumulator from zero; with `out` (a fused step 0) each accumulator
+  // pair of the previous tile is converted and stored right before the step's MFMAs overwrite it, so the
+  // epilogue's VALU work and stores run beside the next tile's first MFMAs instead of stalling the matrix
+  // core.
   auto kstep = [&](int s, __amdgpu_buffer_rsrc_t rc, __amdgpu_buffer_rsrc_t rn, int nb, bool first,
                    const __amdgpu_buffer_rsrc_t* out) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
@@ -434,7 +435,8 @@ hipError_t launch_proj_gemm(const _Float16* X, long long ldx, const _Float16* W,
   // The compile-time-K kernel where one is built (other K: the generic kernel).
   const bool multi = K > kGemmMaxK;
   auto* fk = !blocked || ldc > (1 << 20) ? nullptr
-             : multi                      ? (K % 256 == 0 ? proj_gemm_blocked_kernel<8, true> : proj_gemm_blocked_kernel<4, true>)
+             : multi && K % 256 == 0      ? proj_gemm_blocked_kernel<8, true>
+             : multi                      ? proj_gemm_blocked_kernel<4, true>
              : K == 128                   ? proj_gemm_blocked_kernel<4, false>
              : K == 256                   ? proj_gemm_blocked_kernel<8, false>
              : K == 384                   ? proj_gemm_blocked_kernel<12, false>

@@ -72,7 +72,8 @@ struct Tile {
 // Steps per block of the unrolled step loop: layer 0 moves x a block at a time, and a workgroup looks
 // at its consumer's progress (and reports its own) once per block.
 constexpr int kBlock = 8;
-static_assert(kHandoffSlots % kBlock == 0 && kHandoffSlots >= 3 * kBlock, "the ring covers the layers' lag and a stale report");
+static_assert(kHandoffSlots % kBlock == 0 && kHandoffSlots >= 3 * kBlock,
+              "the ring covers the layers' lag and a stale report");
 
 // LDS of one workgroup.  Layers >= 1 keep the inputs of two steps (step t in slot t & 1), layer 0 those
 // of two blocks.
@@ -176,8 +177,8 @@ __device__ __forceinline__ void wavefront_body(const ForwardArgs& a, WavefrontLd
       for (int q = 0; q < 4; ++q) {
         w[kc][q] = f16x8{};
         if (kc >= KCI)
-          w[kc][q] = reinterpret_cast<const f16x8*>(
-              a.wpack)[((((size_t)layer * 16 + (u >> 3)) * KCR + kc - KCI) * 2 + ((u >> 2) & 1)) * 64 + kg * 16 + (u & 3) * 4 + q];
+          w[kc][q] = reinterpret_cast<const f16x8*>(a.wpack)[
+              ((((size_t)layer * 16 + (u >> 3)) * KCR + kc - KCI) * 2 + ((u >> 2) & 1)) * 64 + kg * 16 + (u & 3) * 4 + q];
         else if (UP)
           w[kc][q] = *reinterpret_cast<const f16x8*>(
               a.wih_up + ((size_t)(layer - 1) * 4 * HP + ((u >> 3) * 4 + (u & 3)) * 8 + 2 * q + ((u >> 2) & 1)) * HP +
