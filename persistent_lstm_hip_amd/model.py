@@ -17,6 +17,7 @@ from __future__ import annotations
 
 import os
 import weakref
+from functools import lru_cache
 from typing import Any, Optional, Sequence, Tuple
 
 import torch
@@ -120,6 +121,13 @@ class _TensorSetKey:
         return True
 
 
+@lru_cache(maxsize=None)
+def _param_names(num_layers: int, bias: bool) -> Tuple[str, ...]:
+    """The attributes that PersistentLSTM packs, layer by layer."""
+    kinds = ("weight_ih", "weight_hh", "bias_ih", "bias_hh") if bias else ("weight_ih", "weight_hh")
+    return tuple(f"{kind}_l{l}" for l in range(num_layers) for kind in kinds)
+
+
 class PersistentLSTM(nn.Module):
     """nn.LSTM-compatible module (batch_first=True, unidirectional, no projection) on the HIP kernel."""
 
@@ -168,9 +176,16 @@ class PersistentLSTM(nn.Module):
         return ext is not None and ext.supports(self.input_size, self.hidden_size, self.num_layers, 0)
 
     def packed_blob(self, device: torch.device, linear: Optional[nn.Linear] = None) -> torch.Tensor:
-        """The device-resident packed weights (re-packed when a parameter or its version changes)."""
-        params = list(self._parameters.values())
-        if len(params) != (4 if self.bias else 2) * self.num_layers:  # e.g. a parametrized weight
+        """The device-resident packed weights (re-packed when a packed tensor or its version changes).
+
+        The key is made of the tensors that are packed: straight from the parameter table while every one of
+        them is a parameter under its own name (an attribute look-up each costs several times that), else, for
+        a weight that something else computes from a parameter of another name (pruning, a spectral or weight
+        norm, a parametrization), through the attributes."""
+        own = self._parameters
+        try:
+            params = [own[name] for name in _param_names(self.num_layers, self.bias)]
+        except KeyError:
             params = [p for l in range(self.num_layers) for p in self.layer_params(l)]
         if linear is not None:
             params += (linear.weight, linear.bias)
