@@ -259,7 +259,8 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
   if (mt >= tiles_m) return;
   const int nblk = M / 16;
   const int xa = (int)(ldx * 32), ca = (int)(ldc * 32);  // bytes from one 16-row block to the next
-  // 16-row blocks a descriptor may span (its byte count is a 31-bit number)
+  // 16-row blocks a descriptor may span (its byte count is a 31-bit number; the launch sees to it that the
+  // wave's four fit)
   const int max_xb = 0x7FFFFFFF / xa, max_cb = 0x7FFFFFFF / ca;
   // X rows of m-tile t held by this wave: blocks 32 t + 4 wave .. + 3
   auto xrs = [&](int t) {
@@ -432,15 +433,19 @@ hipError_t launch_proj_gemm(const _Float16* X, long long ldx, const _Float16* W,
   // m-tile), placed so that an m-group's slices share an XCD.
   const int m_groups = std::max(1, std::min(tiles_m, std::max(cus, 1) / n_slices));
   const int grid = ((m_groups + 7) / 8) * 8 * n_slices;
-  // The compile-time-K kernel where one is built (other K: the generic kernel).
+  // Blocked layouts: a compile-time-K kernel for every K (a multiple of 128).  It addresses a wave's 64 rows of X
+  // and of C by 31-bit byte offsets, so wider ones (ldx from 2^24 on; no layer of a model is) take the
+  // run-time-K kernel, which forms 64-bit addresses.
   const bool multi = K > kGemmMaxK;
-  auto* fk = !blocked || ldc > (1 << 20) ? nullptr
-             : multi && K % 256 == 0      ? proj_gemm_blocked_kernel<8, true>
-             : multi                      ? proj_gemm_blocked_kernel<4, true>
-             : K == 128                   ? proj_gemm_blocked_kernel<4, false>
-             : K == 256                   ? proj_gemm_blocked_kernel<8, false>
-             : K == 384                   ? proj_gemm_blocked_kernel<12, false>
-                                          : proj_gemm_blocked_kernel<16, false>;
+  const bool narrow = ldx <= INT32_MAX / (32 * kGemmWM) && ldc <= (1 << 20);
+  auto* fk = !blocked || !narrow     ? nullptr
+             : multi && K % 256 == 0 ? proj_gemm_blocked_kernel<8, true>
+             : multi                 ? proj_gemm_blocked_kernel<4, true>
+             : K == 128              ? proj_gemm_blocked_kernel<4, false>
+             : K == 256              ? proj_gemm_blocked_kernel<8, false>
+             : K == 384              ? proj_gemm_blocked_kernel<12, false>
+             : K == 512              ? proj_gemm_blocked_kernel<16, false>
+                                     : nullptr;
   if (fk) {
     hipLaunchKernelGGL(fk, dim3(grid), dim3(kGemmThreads), 0, s, X, ldx, W, multi ? K / (K % 256 == 0 ? 256 : 128) : 1, C,
                        ldc, (int)M, tiles_m, n_slices, m_groups);

@@ -105,3 +105,33 @@ def test_blocked_gemm_k_blocks(gpu, rows, k, cols):
     got = gpu.from_blocked(gpu.input_projection(gpu.to_blocked(x), w, blocked=True)).double()
     want = x.double() @ w.double().t()
     assert ((got - want).abs() <= want.abs() * 2.0 ** -11 + 1e-4).all()
+
+
+@pytest.mark.parametrize("k", [256, 640, 768])
+@pytest.mark.parametrize("rows,ldx", [(64, (1 << 24) - 32), (64, 1 << 24), (80, 1 << 25), (64, 1 << 26)])
+def test_blocked_gemm_very_wide_x(gpu, k, rows, ldx):
+    """Blocked x whose 64 rows of a wave end around 2^31 bytes: bit for bit the result of the same columns in a
+    buffer of their own width (both sum an element's products in ascending order of k)."""
+    print(f"[gpu-case] blocked GEMM rows={rows} k={k} ldx={ldx}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = gpu.to_blocked(torch.randn(rows, k, device="cuda", generator=g).half())
+    w = (torch.randn(128, k, device="cuda", generator=g) / k ** 0.5).half()
+    wide = torch.empty(rows, ldx, device="cuda", dtype=torch.float16)  # (columns past k stay unwritten)
+    wide.view(rows // 16, ldx // 32, 512)[:, :k // 32] = x.view(rows // 16, k // 32, 512)
+    got = gpu.input_projection(wide, w, blocked=True)
+    assert torch.equal(got, gpu.input_projection(x, w, blocked=True))
+
+
+@pytest.mark.parametrize("k", [128, 640])
+def test_blocked_gemm_very_wide_result(gpu, k):
+    """More columns than the compile-time-K kernel's offsets cover: the first 2^20 are bit for bit those of a
+    product of that width, the others those of their own product."""
+    n = (1 << 20) + 256
+    print(f"[gpu-case] blocked GEMM cols={n} k={k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x = gpu.to_blocked(torch.randn(32, k, device="cuda", generator=g).half())
+    w = (torch.randn(n, k, device="cuda", generator=g) / k ** 0.5).half()
+    got = gpu.input_projection(x, w, blocked=True).view(2, n // 32, 512)
+    for part in (slice(0, 1 << 20), slice(1 << 20, n)):
+        want = gpu.input_projection(x, w[part], blocked=True).view(2, -1, 512)
+        assert torch.equal(got[:, part.start // 32:part.stop // 32], want)
