@@ -10,10 +10,10 @@
 //
 // Design (a 128-column slice of W over 512 K is 128 KB of LDS):
 //   * weight-stationary: each workgroup owns one 128-column slice of W, loaded once into LDS in MFMA
-//     fragment order when K <= 512 (for K > 512 the slice is held in K blocks of 512, reloaded in
-//     turn for every m-tile between two barriers), and walks the 512-row m-tiles of its m-group; its
-//     8 waves (two per SIMD) each
-//     compute a 64 (m) x 128 (n) sub-tile with v_mfma_f32_16x16x32_f16 (4 x 8 accumulator tiles,
+//     fragment order when K <= 512 (for K > 512 the slice is held in K blocks that take turns in LDS
+//     for every m-tile, between two barriers: of 512 in proj_gemm_kernel, of 256 or 128 with the first
+//     ones kept in proj_gemm_blocked_kernel), and walks the 512-row m-tiles of its m-group; its
+//     8 waves (two per SIMD) each compute a 64 (m) x 128 (n) sub-tile with v_mfma_f32_16x16x32_f16 (4 x 8 accumulator tiles,
 //     128 fp32 per lane), W as the MFMA's A operand and X as its B operand;
 //   * X goes from global memory straight into the B-fragment registers (a lane's 8 consecutive k
 //     of one row are one 16-byte load), through a ring of 4 k-steps of 32: the loads of step s + 3
@@ -37,6 +37,7 @@
 // multiples of 8 (blocked: of 32, and M % 16 == 0), 16-byte aligned pointers.  Rows m >= M are not
 // stored (their loads are clamped to row M - 1).
 #include <algorithm>
+#include <type_traits>
 
 #include "plh_device.h"
 
@@ -218,43 +219,53 @@ proj_gemm_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* 
 // (interleaved runs on one box each); the stores in the next tile's first step: 0.943-0.951 ->
 // 0.933-0.935 ms and 0.105-0.106 -> 0.104-0.106 ms, bit-identical.
 //
-// MULTI: the W slice does not fit the LDS, so it is held one K block at a time, and the tiles take their blocks in
-// alternating order (up, down, up, ..): the block left by one tile is the next one's first, so a tile reloads
-// blocks - 1 of them, moved from global memory to LDS directly (16 bytes per lane, no registers).  Against the
-// run-time-K kernel, which reloads blocks of 512 twice per tile: [128000,1024]x[1024,4096] 1.10-1.16 -> 0.97-1.01
-// ms, K = 768 0.84-0.86 -> 0.71 ms, K = 640 0.73 -> 0.64 ms.  Blocks of 512 (the largest that fit) spilled 21 VGPRs
-// (+3%); two buffers, the next block loading under the current one's MFMAs, were 2-6% slower.
+// MULTI: the W slice does not fit the LDS.  Its first KEEP blocks stay there (K = 1024: one of 256; odd multiples of
+// 128: three of 128), the others are reloaded for every tile, from global memory to LDS directly (16 bytes per
+// lane, no registers).  Every tile takes its blocks in ascending order, so a row's sums do not depend on the
+// tile it stands in: equal rows have equal results, and the bits are those of the run-time-K kernel.  (Walking
+// the blocks up and down, with the block left by one tile the next one's first, reloads as many at K above 640
+// but summed odd and even tiles in opposite orders; reloading all of them in ascending order took 1.02, 0.79
+// and 0.64 ms where the alternation took 0.93, 0.69 and 0.61.)  Interleaved on one box, the alternation -> this:
+// [128000,1024]x[1024,4096] 0.985-0.999 -> 0.996-1.003 ms, K = 768 0.732-0.734 -> 0.729-0.731, K = 640 0.641-0.643
+// -> 0.572-0.573; the run-time-K kernel, which reloads blocks of 512 twice per tile: 1.06, 0.82 and 0.71 on a
+// box where the alternation took 0.93, 0.69 and 0.61.  Blocks of 512 spilled 21 VGPRs (+3%); two buffers, the
+// next block loading under the current one's MFMAs, were 2-6% slower.
 template <int KS, bool MULTI>
 __global__ void __launch_bounds__(kGemmThreads)
 proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* __restrict__ W, int blocks,
                          _Float16* __restrict__ C, long long ldc, int M, int tiles_m, int n_slices, int m_groups) {
   static_assert(kGemmWaves == 8 && kGemmWM == 4 && KS % kRing == 0 && KS * 32 <= kGemmMaxK, "tile shape");
   const int K = MULTI ? 32 * KS * blocks : 32 * KS;
-  __shared__ f16x8 wl[KS * 8 * 64];  // [k-chunk][n-tile 0..7][64 lanes] f16x8
+  // MULTI: blocks 0 .. KEEP - 1 stay in LDS for good (slots 1 .. KEEP), the others take turns in slot 0.
+  constexpr int KEEP = MULTI ? kGemmKbSteps / KS - 1 : 0;
+  static_assert(!MULTI || KEEP >= 1, "a tile's first block is one that stays");
+  constexpr int kSlotVec = KS * 8 * 64;  // f16x8 of one block: [k-chunk][n-tile 0..7][64 lanes]
+  __shared__ f16x8 wl[(KEEP + 1) * kSlotVec];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   const int ns = idx % n_slices;
   const int mg = (idx / n_slices) * 8 + xcd;
   if (mg >= m_groups) return;
   const int n0 = ns * kGemmBN;
-  // K block b of the W slice into LDS (the caller's barriers around it): wave w loads n-tile w of every k-chunk.
+  // K block b of the W slice into a slot (the caller's barriers around it): wave w loads n-tile w of every
+  // k-chunk, through registers or from global memory to LDS directly.
   const _Float16* const wsrc = W + (size_t)(n0 + gemm_w_row(wave, lane & 15)) * K + (lane >> 4) * 8;
-  auto load_w = [&](int b) {
+  auto load_w = [&](int b, int slot, auto direct) {
     const _Float16* const src = wsrc + b * (KS * 32);
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
-      f16x8* const dst = wl + (i * 8 + wave) * 64;
-      if constexpr (!MULTI)
+      f16x8* const dst = wl + slot * kSlotVec + (i * 8 + wave) * 64;
+      if constexpr (!decltype(direct)::value)
         dst[lane] = *reinterpret_cast<const f16x8*>(src + i * 32);
       else
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(uintptr_t)(src + i * 32),
                                          (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
     }
-    if constexpr (MULTI) wait_vmem_all();
+    if constexpr (decltype(direct)::value) wait_vmem_all();
   };
-  load_w(0);
+#pragma unroll
+  for (int b = 0; b < (MULTI ? KEEP : 1); ++b) load_w(b, MULTI ? 1 + b : 0, std::false_type());
   __syncthreads();
-  int kb = 0, dir = 1;  // the K block in LDS, and the order of this tile's blocks
   int mt = mg;
   if (mt >= tiles_m) return;
   const int nblk = M / 16;
@@ -294,8 +305,10 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
   // pair of the previous tile is converted and stored right before the step's MFMAs overwrite it, so the
   // epilogue's VALU work and stores run beside the next tile's first MFMAs instead of stalling the matrix
   // core.
-  auto kstep = [&](int s, __amdgpu_buffer_rsrc_t rc, __amdgpu_buffer_rsrc_t rn, int nb, bool first,
+  auto kstep = [&](int s, int kb, __amdgpu_buffer_rsrc_t rc, __amdgpu_buffer_rsrc_t rn, int nb,
                    const __amdgpu_buffer_rsrc_t* out) __attribute__((always_inline)) {
+    const bool first = kb == 0;
+    const f16x8* const wk = wl + (kb < KEEP ? 1 + kb : 0) * kSlotVec + lane;
     __builtin_amdgcn_sched_barrier(0);
     {
       const int sn = s + kRing - 1;  // this tile's step sn, or the next tile's first steps
@@ -305,11 +318,11 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
         ld(rn, nb * KS + sn - KS, xr[sn % kRing]);
     }
     f16x8 wa[3];
-    wa[0] = wl[(s * 8 + 0) * 64 + lane];
-    wa[1] = wl[(s * 8 + 1) * 64 + lane];
+    wa[0] = wk[(s * 8 + 0) * 64];
+    wa[1] = wk[(s * 8 + 1) * 64];
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
-      if (b + 2 < 8) wa[(b + 2) % 3] = wl[(s * 8 + b + 2) * 64 + lane];
+      if (b + 2 < 8) wa[(b + 2) % 3] = wk[(s * 8 + b + 2) * 64];
       if (out && b % 2 == 0) {
         // the previous tile's column blocks n0 / 32 + b / 2: blocks 32 mt + 4 wave + a
 #pragma unroll
@@ -373,28 +386,25 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
     const int nmt = mt + m_groups;
     const int pmt = nmt < tiles_m ? nmt : mt;  // prefetch target past the last tile: reload this one
     const auto rc = xrs(mt), rn = xrs(pmt);
-    if constexpr (!MULTI) {
-      kstep(0, rc, rn, 0, true, &prev);
+    // block 0; what follows it in the X ring: the tile's next block, or the next tile
+    kstep(0, 0, rc, MULTI ? rc : rn, MULTI ? 1 : 0, &prev);
 #pragma unroll
-      for (int s = 1; s < KS; ++s) kstep(s, rc, rn, 0, true, nullptr);
-    } else {
-      kstep(0, rc, rc, kb + dir, true, &prev);
-#pragma unroll
-      for (int s = 1; s < KS; ++s) kstep(s, rc, rc, kb + dir, true, nullptr);
+    for (int s = 1; s < KS; ++s) kstep(s, 0, rc, MULTI ? rc : rn, MULTI ? 1 : 0, nullptr);
+    if constexpr (MULTI) {
 #pragma unroll 1
-      for (int j = 1; j < blocks; ++j) {
-        // every wave is done with the block (its MFMAs read it from registers loaded before them)
-        __syncthreads();
-        kb += dir;
-        load_w(kb);
-        __syncthreads();
-        const bool more = j + 1 < blocks;
+      for (int kb = 1; kb < blocks; ++kb) {
+        if (kb >= KEEP) {
+          // every wave is done with the slot (its MFMAs read it from registers loaded before them)
+          __syncthreads();
+          load_w(kb, 0, std::true_type());
+          __syncthreads();
+        }
+        const bool more = kb + 1 < blocks;
         const auto rx = more ? rc : rn;
-        const int nb = more ? kb + dir : kb;
+        const int nb = more ? kb + 1 : 0;
 #pragma unroll
-        for (int s = 0; s < KS; ++s) kstep(s, rc, rx, nb, false, nullptr);
+        for (int s = 0; s < KS; ++s) kstep(s, kb, rc, rx, nb, nullptr);
       }
-      dir = -dir;
     }
     __builtin_amdgcn_sched_barrier(0);
     prev = crs(mt);

@@ -135,3 +135,19 @@ def test_blocked_gemm_very_wide_result(gpu, k):
     for part in (slice(0, 1 << 20), slice(1 << 20, n)):
         want = gpu.input_projection(x, w[part], blocked=True).view(2, -1, 512)
         assert torch.equal(got[:, part.start // 32:part.stop // 32], want)
+
+
+@pytest.mark.parametrize("k", [512, 640, 768, 896, 1024])
+def test_a_row_of_the_blocked_gemm_does_not_depend_on_its_place(gpu, k):
+    """Three row tiles per workgroup (32 column slices leave 8 workgroups of rows, 17 tiles and a part of one): a
+    row's sums run over k in ascending order wherever it stands, so equal rows have equal results, bit for bit,
+    and those of the row-major kernel."""
+    print(f"[gpu-case] blocked GEMM equal rows k={k}", flush=True)
+    rows, cols = 512 * 17 + 48, 4096
+    g = torch.Generator(device="cuda").manual_seed(k)
+    few = torch.randn(3, k, device="cuda", generator=g).half()
+    w = (torch.randn(cols, k, device="cuda", generator=g) / k ** 0.5).half()
+    which = torch.arange(rows, device="cuda") % 3
+    got = gpu.from_blocked(gpu.input_projection(gpu.to_blocked(few[which]), w, blocked=True))
+    assert torch.equal(got, got[:3][which])
+    assert torch.equal(got[:3], gpu.input_projection(few, w))
