@@ -31,7 +31,7 @@ int fail_hip(hipError_t e, const char* what) {
   return fail(PLH_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// Co-resident workgroup capacity per (device, HP, tile rows, path), queried once.
+// Co-resident workgroup capacity per device and set of kernel variants (plh::capacity_key), queried once.
 std::mutex g_cap_mu;
 std::unordered_map<long long, int> g_cap;
 
@@ -39,7 +39,7 @@ int capacity(const plh::Geometry& g, int tile_rows, hipError_t* err) {
   int dev = 0;
   *err = hipGetDevice(&dev);
   if (*err != hipSuccess) return 0;
-  const long long key = (((long long)dev * 4096 + g.HP) * 64 + tile_rows) * 2 + g.rec;
+  const long long key = plh::capacity_key(dev, g, tile_rows);
   {
     std::lock_guard<std::mutex> lk(g_cap_mu);
     auto it = g_cap.find(key);

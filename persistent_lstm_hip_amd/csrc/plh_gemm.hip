@@ -13,8 +13,8 @@
 //     fragment order when K <= 512 (for K > 512 the slice is held in K blocks that take turns in LDS
 //     for every m-tile, between two barriers: of 512 in proj_gemm_kernel, of 256 or 128 with the first
 //     ones kept in proj_gemm_blocked_kernel), and walks the 512-row m-tiles of its m-group; its
-//     8 waves (two per SIMD) each compute a 64 (m) x 128 (n) sub-tile with v_mfma_f32_16x16x32_f16 (4 x 8 accumulator tiles,
-//     128 fp32 per lane), W as the MFMA's A operand and X as its B operand;
+//     8 waves (two per SIMD) each compute a 64 (m) x 128 (n) sub-tile with v_mfma_f32_16x16x32_f16
+//     (4 x 8 accumulator tiles, 128 fp32 per lane), W as the MFMA's A operand and X as its B operand;
 //   * X goes from global memory straight into the B-fragment registers (a lane's 8 consecutive k
 //     of one row are one 16-byte load), through a ring of 4 k-steps of 32: the loads of step s + 3
 //     are issued before the MFMAs of step s, across tile boundaries, so a load has three steps
@@ -223,7 +223,7 @@ proj_gemm_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* 
 // 128: three of 128), the others are reloaded for every tile, from global memory to LDS directly (16 bytes per
 // lane, no registers).  Every tile takes its blocks in ascending order, so a row's sums do not depend on the
 // tile it stands in: equal rows have equal results, and the bits are those of the run-time-K kernel.  (Walking
-// the blocks up and down, with the block left by one tile the next one's first, reloads as many at K above 640
+// the blocks up and down, with the block left by one tile the next one's first, reloads as many blocks of 256
 // but summed odd and even tiles in opposite orders; reloading all of them in ascending order took 1.02, 0.79
 // and 0.64 ms where the alternation took 0.93, 0.69 and 0.61.)  Interleaved on one box, the alternation -> this:
 // [128000,1024]x[1024,4096] 0.985-0.999 -> 0.996-1.003 ms, K = 768 0.732-0.734 -> 0.729-0.731, K = 640 0.641-0.643

@@ -179,6 +179,11 @@ hipError_t launch_repeat_first_row(const _Float16* in, _Float16* out, int rows, 
 const void* wavefront_kernel(int HP, int tile_rows, bool ragged, bool wide);
 const void* sliced_kernel(int HP, int wg_tiles);
 
+// Names the set of kernel variants whose co-residency recurrent_capacity looks up on device `dev`: geometries
+// that run different kernels have different keys.
+inline long long capacity_key(int dev, const Geometry& g, int tile_rows) {
+  return (((((long long)dev * 4096 + g.HP) * 64 + tile_rows) * 2 + g.rec) * 2 + g.wide_ok) * 2 + g.rec_x0;
+}
 // Co-resident workgroups of the persistent kernel on the current device (0 with *err set on error).
 int recurrent_capacity(const Geometry& g, int tile_rows, hipError_t* err);
 hipError_t launch_recurrent(const Geometry& g, const ForwardArgs& a, hipStream_t s);
