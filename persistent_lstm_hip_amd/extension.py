@@ -624,6 +624,9 @@ def load_extension() -> Optional[NativeLibrary]:
     except OSError as exc:
         _load_error = f"cannot load {LIB_PATH}: {exc}"
         return None
+    except AttributeError as exc:  # built before a function this front end binds was added
+        _load_error = f"{LIB_PATH} is out of date ({exc}): run `python -m persistent_lstm_hip_amd.build`"
+        return None
 
 
 def load_error() -> Optional[str]:

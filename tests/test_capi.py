@@ -235,3 +235,24 @@ def test_kernel_timing_arming_without_forwards(ext):
     ms, n = ext.kernel_timing_read()
     assert n == 0 and ms == 0.0
     assert ext.lib.plh_kernel_timing(-1) == PLH_ERR_INVALID
+
+
+def test_a_library_without_a_newer_function_is_a_reason_not_an_exception(tmp_path, monkeypatch):
+    """An older build of the same ABI number lacks functions added since: load_extension() is None, with the
+    missing function named in load_error()."""
+    import shutil
+
+    from persistent_lstm_hip_amd import extension
+
+    cc = shutil.which("gcc") or shutil.which("cc") or shutil.which("clang")
+    if cc is None:
+        pytest.skip("no C compiler")
+    absent = {"plh_detects_uniform", "plh_forward_detect"}
+    src = "".join(f"int {n}(void) {{ return 1; }}\n" for n in declared_functions() if n not in absent)
+    (tmp_path / "old.c").write_text(src)
+    lib = str(tmp_path / "libold.so")
+    subprocess.run([cc, "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", lib], check=True)
+    monkeypatch.setattr(extension, "LIB_PATH", lib)
+    monkeypatch.setattr(extension, "_load_error", None)
+    assert extension.load_extension.__wrapped__() is None
+    assert "plh_detects_uniform" in extension.load_error() and "persistent_lstm_hip_amd.build" in extension.load_error()
