@@ -346,7 +346,11 @@ class NativeLibrary:
     def forward_detect(self, packed: torch.Tensor, dims: Sequence[int], x: torch.Tensor) -> torch.Tensor:
         """plh_forward_detect: the head outputs [B, O] of full-length rows x [B, T, I] on a HIP device."""
         I, H, L, O = dims
+        if not isinstance(x, torch.Tensor) or x.dim() != 3:
+            raise ValueError("x must be a [batch, seq_len, input_size] tensor")
         device = x.device
+        if device.type != "cuda":
+            raise ValueError("x must be on a HIP device: this library has no CPU path")
         if int(x.size(2)) != I:
             raise ValueError(f"x has input size {int(x.size(2))}, the model expects {I}")
         if not x.is_floating_point():

@@ -256,3 +256,12 @@ def test_a_library_without_a_newer_function_is_a_reason_not_an_exception(tmp_pat
     monkeypatch.setattr(extension, "_load_error", None)
     assert extension.load_extension.__wrapped__() is None
     assert "plh_detects_uniform" in extension.load_error() and "persistent_lstm_hip_amd.build" in extension.load_error()
+
+
+@pytest.mark.parametrize("shape,message", [((2, 3, 5), "HIP device"), ((3, 5), "batch, seq_len, input_size")])
+def test_forward_detect_checks_its_input(ext, shape, message):
+    """As forward: host memory must not reach a kernel."""
+    import torch
+
+    with pytest.raises(ValueError, match=message):
+        ext.forward_detect(torch.zeros(256, dtype=torch.uint8), (5, 128, 4, 24), torch.zeros(*shape).half())
