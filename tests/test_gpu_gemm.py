@@ -93,11 +93,13 @@ def test_input_projection_rejects_bad_shapes(gpu):
             gpu.input_projection(z(*xs), z(*ws))
 
 
-@pytest.mark.parametrize("rows,k,cols", [(16, 640, 128), (528, 768, 256), (8208, 896, 128), (1040, 1024, 384), (32, 2176, 128)])
+@pytest.mark.parametrize("rows,k,cols", [(16, 640, 128), (528, 768, 256), (8208, 896, 128), (1040, 1024, 384),
+                                         (32, 2176, 128), (9248, 640, 4096), (9248, 896, 4096), (9248, 768, 4096),
+                                         (9248, 1024, 4096), (9248, 1152, 4096)])
 def test_blocked_gemm_k_blocks(gpu, rows, k, cols):
-    """K above 512 in blocks of 256 or 128, taken in alternating order by successive row tiles: one tile, a
-    tile and a remainder, several tiles per workgroup; an odd and an even number of blocks.  fp16 results of
-    fp32 sums: half an ulp (2^-11 of the value) plus the sums' own rounding."""
+    """K above 512 in blocks of 256 or 128: one row tile, a tile and a remainder, and (4096 columns, which leave 8
+    workgroups of rows for 19 tiles) up to three tiles per workgroup; an odd and an even number of blocks.  fp16
+    results of fp32 sums: half an ulp (2^-11 of the value) plus the sums' own rounding."""
     print(f"[gpu-case] blocked GEMM rows={rows} k={k} cols={cols}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(k)
     x = torch.randn(rows, k, device="cuda", generator=g).half()

@@ -109,10 +109,17 @@ def test_wide_inputs(gpu, I, H, L, B, T):
         assert np.abs(res["h_n"].float().cpu().numpy()[:, rows] - want["h_n"]).max() <= 2 * BOUND
 
 
+def _verdict_end(L, B):
+    """End of the status and counter words of a wavefront forward in 8-row tiles: 256 bytes, then a word per
+    (layer, tile), rounded up to 256 bytes."""
+    return 256 + (4 * L * ((B + 7) // 8) + 255) // 256 * 256
+
+
 @pytest.mark.parametrize("I,H,L,B,T", [(5, 128, 4, 512, 60), (1, 20, 1, 2, 1), (9, 64, 2, 33, 17), (128, 128, 2, 9, 40)])
 def test_equal_rows_found_on_the_device(gpu, monkeypatch, I, H, L, B, T):
     """Equal rows, and equal but for one element (the last one, the first one of row 1, the middle of a row):
-    the outputs are bit for bit those of a forward without detection."""
+    the outputs are bit for bit those of a forward without detection, and the verdict words (behind the status
+    word, one per block of the prologue) are all zero for equal rows and only for them."""
     print(f"[gpu-case] uniform I={I} H={H} L={L} B={B} T={T}", flush=True)
     model = PersistentLSTMRegressor.from_native_module(make_regressor(I, H, L, 11)).to("cuda").half().eval()
     assert gpu.detects_uniform((I, H, L, 11), B, T, torch.device("cuda"))
@@ -122,29 +129,35 @@ def test_equal_rows_found_on_the_device(gpu, monkeypatch, I, H, L, B, T):
         if where is not None and where[0] > 0:
             x[where] += 1
         monkeypatch.setenv("PERSISTENT_LSTM_HIP_UNIFORM_BATCH", "auto")
+        model(x)  # (a workspace large enough exists from here on)
+        words = gpu.workspace(x.device, 256)[:_verdict_end(L, B)].view(torch.int32)[1:]
+        words.fill_(-1)  # nothing reads them before the prologue has written its own
         got = model(x)
         gpu.check_status(torch.device("cuda"))
+        written = words[words != -1]
+        assert written.numel() > 0 and torch.equal(words[:written.numel()], written)
+        assert bool((written != 0).any()) == (where is not None and where[0] > 0), where
         monkeypatch.setenv("PERSISTENT_LSTM_HIP_UNIFORM_BATCH", "0")
         assert torch.equal(got, model(x)), where
 
 
-@pytest.mark.parametrize("I,H,L,B,T", [
-    (5, 128, 4, 1060, 40),    # 1024 rows in 16-row tiles, 36 in 8-row tiles
-    (5, 200, 4, 530, 12),     # two tiles per workgroup, then one
-    (5, 400, 4, 540, 12),     # layer by layer, then all layers at once
-    (300, 256, 2, 1030, 5),   # layer by layer twice
-    (5, 600, 2, 140, 6),      # padded H 1024: 128 rows, then 12
+@pytest.mark.parametrize("I,H,L,B,T,edge", [
+    (5, 128, 4, 1060, 40, 1024),    # 1024 rows in 16-row tiles, 36 in 8-row tiles
+    (5, 200, 4, 530, 12, 512),      # two tiles per workgroup, then one
+    (5, 400, 4, 540, 12, 512),      # layer by layer, then all layers at once
+    (300, 256, 2, 1030, 5, 1024),   # layer by layer twice
+    (5, 600, 2, 140, 6, 128),       # padded H 1024: 128 rows, then 12
 ])
-def test_rows_after_the_last_full_launch(gpu, I, H, L, B, T):
-    """A forward in several launches whose last one takes another plan: rows of both against the oracle
-    (layer-sequential rows also round their projections, as above), states and sequence included."""
+def test_rows_after_the_last_full_launch(gpu, I, H, L, B, T, edge):
+    """A forward in several launches whose last one takes another plan: rows on both sides of the `edge` between
+    them against the oracle (layer-sequential rows also round their projections, as above), states and sequence
+    included."""
     print(f"[gpu-case] remainder I={I} H={H} L={L} B={B} T={T}", flush=True)
     native = make_regressor(I, H, L, 3)
     x = make_x(B, T, I, seed=8)
     out, (h, c) = _lstm(native)(x.to("cuda", torch.float16))
     gpu.check_status(torch.device("cuda"))
-    mid = 508 if B > 516 else 124
-    rows = np.unique(np.r_[0:4, mid:mid + 8, B - 12:B])
+    rows = np.unique(np.r_[0:4, edge - 6:min(edge + 8, B), B - 4:B])
     want = _oracle(native, x[rows])
     assert np.abs(out.float().cpu().numpy()[rows] - want["out_seq"]).max() <= 2 * BOUND
     assert np.abs(h.float().cpu().numpy()[:, rows] - want["h_n"]).max() <= 2 * BOUND
