@@ -67,10 +67,12 @@ struct Plan {
   bool fits = true;  // the workgroups of one tile fit the device at once
   bool pad8 = false; // the co-resident tiles are a multiple of 8: a launch may round its grid up to 8 tiles
   int cap_wgs = 0;   // co-resident workgroups of the plan's tile size
+  int cap8 = 0;      // ... of 8-row tiles (wavefront kernel)
 };
 
 Plan make_plan(const plh::Geometry& g, int batch, int cap8, int cap16) {
   Plan p;
+  p.cap8 = cap8;
   batch = std::max(batch, 1);
   const int tiles8 = (batch + 7) / 8;
   if (g.slices == 1 && (long long)g.L * tiles8 <= cap8) {
@@ -119,9 +121,34 @@ Plan plan_path(const plh::Geometry& g, int batch, bool need_device, hipError_t* 
 // used whenever one tile of all L layers does not fit the device (L x 16 slices > the co-resident
 // workgroups: more than 16 layers at padded H 512).
 constexpr size_t kMaxSeqWorkspace = (size_t)24 << 30;
-Plan plan_for(const plh::Geometry& g, int batch, int seq_len, bool need_device, hipError_t* err) {
+
+// Inputs wider than padded H 128, whose batch takes several wavefront launches (`full` of plan p's rows, then one of
+// `rest`): whether those are faster than the layer-sequential path in launches of q's rows, by the time of a launch
+// of each kind in us, fitted to measurements.  A wavefront launch starts, fills its layers' pipeline and runs T
+// steps (shorter ones in 8-row tiles, where the rows allow them); the other runs T steps of every layer, with
+// a GEMM of all its rows in front of each.  Measured at I 300, H 128, everything included: a wavefront launch of
+// 2 layers and 2048 rows, 6 and 640, 8 and 512: 50, 66, 75 at T 8, 105, 99, 115 at T 32; layer by layer, 2048 rows
+// of 2, 6 and 8 layers: 85, 207, 267 and 192, 440, 567.  So several launches lose on short sequences of many
+// layers (6 layers, 2048 rows, T 8: 255 in four launches) and win elsewhere (T 32: 377 against 440).
+bool wide_launches_pay(const plh::Geometry& g, const Plan& p, const Plan& q, int batch, int seq_len) {
+  const int full = batch / p.chunk_rows, rest = batch % p.chunk_rows;
+  if (full + (rest > 0) <= 1) return true;
+  const double L = g.L, T = seq_len;
+  const auto launch = [&](int rows) { return 24 + 5.4 * L + T * (1.1 + 0.5e-3 * rows); };
+  double wave = full * launch(p.chunk_rows);
+  if (rest > 0)
+    wave += (long long)g.L * ((rest + 7) / 8) <= p.cap8 ? 24 + 4.5 * (L - 1) + T * (0.85 + 0.5e-3 * rest)
+                                                        : launch(rest);
+  const int launches = (batch + q.chunk_rows - 1) / q.chunk_rows;
+  return wave <= launches * (23 + L * (15 + 1.25 * T)) + L * T * 0.45e-3 * batch;
+}
+
+// layout_rows: rows of the layer-sequential workspace layout that the caller has laid out already (the rows after
+// the last full launch); 0: the layout is the plan's own.
+Plan plan_for(const plh::Geometry& g, int batch, int seq_len, bool need_device, hipError_t* err, int layout_rows = 0) {
   if (!g.wave_ok) {
-    // Padded H 1024, or an input wider than the padded H: only the layer-sequential path exists.
+    // Padded H 1024, or an input wider than the padded H: the layer-sequential path, or at padded H 128 the
+    // wavefront kernel on layer 0's GEMM projections.
     const plh::Geometry gr = plh::as_layer_sequential(g);
     Plan q = plan_path(gr, batch, need_device, err);
     q.rec = true;
@@ -130,16 +157,18 @@ Plan plan_for(const plh::Geometry& g, int batch, int seq_len, bool need_device, 
       // at once without an exchange per step; the layer-sequential kernel runs them one after another,
       // 1.3 us per step against 0.6-0.8 (I300 H128 L2 B64 T200: 578 -> 180 us).  It runs in the same workspace,
       // its hand-off rings in the place of the layer sequences: where they do not fit there (more than
-      // three layers on a short sequence), and on a device that cannot hold a tile of all layers, the
-      // layer-sequential path serves the call.
+      // three layers on a short sequence), where several launches of it would take longer, and on a device that
+      // cannot hold a tile of all layers, the layer-sequential path serves the call.
       Plan p = plan_path(g, batch, need_device, err);
       if (*err != hipSuccess) return q;
-      p.chunk_rows = std::min(p.chunk_rows, q.chunk_rows);
+      const int rows = std::max(q.chunk_rows, layout_rows);
+      p.chunk_rows = std::min(p.chunk_rows, rows);
       const size_t tiles = (size_t)p.chunk_rows / p.tile_rows;
       const size_t rings = (size_t)(g.L - 1) * p.chunk_rows * std::min(seq_len, plh::kHandoffSlots) * g.HP * 2 +
                            (size_t)g.L * tiles * plh::kCounterStride * 4;
-      if (p.fits && rings <= (size_t)2 * seq_len * q.chunk_rows * g.HP * sizeof(_Float16)) {
-        p.wide_rows = q.chunk_rows;
+      if (p.fits && rings <= (size_t)2 * seq_len * rows * g.HP * sizeof(_Float16) &&
+          wide_launches_pay(g, p, q, batch, seq_len)) {
+        p.wide_rows = rows;
         return p;
       }
     }
@@ -485,10 +514,12 @@ int forward_impl(const void* packed_dev, int input_size, int hidden_size, int nu
       // laid out for the whole: 8-row tiles, one tile per workgroup, or the sliced path instead of the
       // layer-sequential one (kernels of H128 L4 B1500 T250, 1024 + 476 rows: 617 -> 514 us; four layers of
       // 500 steps at H256 B700 2.75 -> 2.08 ms, at H512 B600 8.69 -> 7.17 ms).
-      const Plan rest = plan_for(base, batch - row0, seq_len, true, &err);
+      const Plan rest = plan_for(base, batch - row0, seq_len, true, &err, plan.wide_rows);
       if (err != hipSuccess) return fail_hip(err, "occupancy query");
       const plh::WorkspaceLayout wr = plan_layout(base, rest, seq_len);
-      if (rest.fits && wr.total <= ws_total) {
+      // (Wide inputs: all rows of a batch go layer by layer or none does, so that their projections are rounded
+      // alike; the rings of the rest have the room of the whole.)
+      if (rest.fits && wr.total <= ws_total && !(plan.rec && rest.wide_rows)) {
         plan = rest;
         w = wr;
         g = plan.rec ? plh::as_layer_sequential(base) : base;

@@ -161,3 +161,32 @@ def test_rows_after_the_last_full_launch(gpu, I, H, L, B, T, edge):
     want = _oracle(native, x[rows])
     assert np.abs(out.float().cpu().numpy()[rows] - want["out_seq"]).max() <= 2 * BOUND
     assert np.abs(h.float().cpu().numpy()[:, rows] - want["h_n"]).max() <= 2 * BOUND
+
+
+@pytest.mark.parametrize("I,H,L,B,T,lengths", [
+    (300, 128, 3, 1500, 8, False),    # 1280 rows and 220 in the workspace of all
+    (300, 60, 8, 800, 100, True),     # 512 and 288
+    (150, 128, 6, 2100, 8, False),    # four launches on a short sequence: layer by layer
+    (150, 128, 6, 2100, 40, True),    # ... and all layers at once
+    (129, 128, 8, 4300, 9, False),    # more rows than a layer-by-layer launch holds
+])
+def test_wide_inputs_in_several_launches(gpu, I, H, L, B, T, lengths):
+    """Wide inputs whose batch takes several launches: every row is computed by the same kernels (their projections
+    are rounded alike), so equal rows are equal bit for bit on both sides of every launch boundary; the first ones
+    against the oracle (bound as in test_wide_inputs)."""
+    print(f"[gpu-case] wide launches I={I} H={H} L={L} B={B} T={T}", flush=True)
+    native = make_regressor(I, H, L, 3)
+    few = make_x(3, T, I, seed=7)
+    lens = torch.tensor([T, T // 2, T - 1])
+    which = torch.arange(B) % 3
+    model = _lstm(native)
+    blob = model.packed_blob(torch.device("cuda", torch.cuda.current_device()))
+    res = gpu.forward(blob, (I, H, L, 0), few.to("cuda", torch.float16)[which.cuda()],
+                      lengths=lens[which] if lengths else None, want_out=False, want_seq=True, want_state=True,
+                      check_status=True)
+    for key, dim in (("out_seq", 0), ("h_n", 1), ("c_n", 1)):
+        same = torch.equal(res[key], res[key].index_select(dim, which.cuda()))
+        assert same, key
+    want = _oracle(native, few, lengths=lens.numpy() if lengths else None)
+    assert np.abs(res["out_seq"][:3].float().cpu().numpy() - want["out_seq"]).max() <= 2 * BOUND
+    assert np.abs(res["h_n"][:, :3].float().cpu().numpy() - want["h_n"]).max() <= 2 * BOUND
