@@ -103,9 +103,10 @@ int64_t plh_workspace_bytes(int input_size, int hidden_size, int num_layers, int
  * fp16 before the recurrent sum, as the reference's generic path does (persistent_lstm_hip.cu:
  * 2988-2994); the all-layers path keeps it in fp32, so at padded H 512 the batch size decides which
  * of the two roundings a row gets (both are within the tolerance; the rows after the last full launch of
- * a batch take the path of a batch of their number).  At padded H 128 an input wider than that has its
- * layer-0 projections from the same GEMM, rounded to fp16, in front of launches of all layers (short
- * sequences of more than three layers, or of many layers in several launches: layer by layer).
+ * a batch take the all-layers path where that is faster for their number).  At padded H 128 an input
+ * wider than that has its layer-0 projections from the same GEMM, rounded to fp16, in front of launches
+ * of all layers (short sequences of more than three layers, or of many layers in several launches:
+ * layer by layer).
  * Replaces persistent_lstm4_forward_interleaved (bindings.cpp:157, persistent_lstm_hip.cu:2126-2254)
  * and persistent_lstm_regressor_forward_generic_projected (bindings.cpp:163,
  * persistent_lstm_hip.cu:2923-3181), whose signatures return only the [batch, O] head output;

@@ -186,6 +186,18 @@ Plan plan_for(const plh::Geometry& g, int batch, int seq_len, bool need_device, 
   return n_wave > g.L ? q : p;
 }
 
+// The rows after the last full layer-sequential launch (padded H 512) on the sliced kernel, which plan `rest` runs
+// in n launches: whether that is faster than layer by layer, by the time of a launch of each kind in us, fitted to
+// measurements.  A sliced launch of all layers: 52-66 at T 8, 136 at T 50, 310 at T 150 (L = 4); a layer-sequential
+// layer of as few rows: 27, 90 and 235 (the first), 34, 100 and 270 (the others, with their GEMM).  512 + rest rows,
+// L = 4, rest 64, 128, 192 and 256 (1 to 4 launches), against layer by layer: T 8 0.76, 0.97, 1.20 and 1.41 of its
+// time, T 50 0.74, 0.88, 1.01 and 1.16, T 500 0.67, 0.82, 0.94 and 1.05; one layer is always slower (1.05-1.10).
+bool rest_sliced_pays(const plh::Geometry& g, const Plan& rest, int rows, int seq_len) {
+  const double L = g.L, T = seq_len;
+  const int n = (rows + rest.chunk_rows - 1) / rest.chunk_rows;
+  return n * (5 + 13.5 * L + 1.75 * T) < 15 + 1.48 * T + (L - 1) * (22 + 1.7 * T);
+}
+
 // The workspace layout a plan runs in.
 plh::WorkspaceLayout plan_layout(const plh::Geometry& g, const Plan& p, int seq_len) {
   if (p.wide_rows) return plh::workspace_layout(plh::as_layer_sequential(g), seq_len, p.wide_rows, 16);
@@ -511,15 +523,17 @@ int forward_impl(const void* packed_dev, int input_size, int hidden_size, int nu
   for (int row0 = 0; row0 < batch; row0 = a.row_end) {
     if (row0 > 0 && batch - row0 < plan.chunk_rows) {
       // The rows after the last full launch take the plan of a batch of their size, within the workspace
-      // laid out for the whole: 8-row tiles, one tile per workgroup, or the sliced path instead of the
-      // layer-sequential one (kernels of H128 L4 B1500 T250, 1024 + 476 rows: 617 -> 514 us; four layers of
-      // 500 steps at H256 B700 2.75 -> 2.08 ms, at H512 B600 8.69 -> 7.17 ms).
+      // laid out for the whole: 8-row tiles, one tile per workgroup, or, where it is faster, the sliced path
+      // instead of the layer-sequential one (kernels of H128 L4 B1500 T250, 1024 + 476 rows: 617 -> 514 us; four
+      // layers of 500 steps at H256 B700 2.75 -> 2.08 ms, at H512 B600 8.69 -> 7.17 ms).
       const Plan rest = plan_for(base, batch - row0, seq_len, true, &err, plan.wide_rows);
       if (err != hipSuccess) return fail_hip(err, "occupancy query");
       const plh::WorkspaceLayout wr = plan_layout(base, rest, seq_len);
       // (Wide inputs: all rows of a batch go layer by layer or none does, so that their projections are rounded
       // alike; the rings of the rest have the room of the whole.)
-      if (rest.fits && wr.total <= ws_total && !(plan.rec && rest.wide_rows)) {
+      const bool pays = !plan.rec || rest.rec ||
+                        (!rest.wide_rows && rest_sliced_pays(base, rest, batch - row0, seq_len));
+      if (rest.fits && wr.total <= ws_total && pays) {
         plan = rest;
         w = wr;
         g = plan.rec ? plh::as_layer_sequential(base) : base;

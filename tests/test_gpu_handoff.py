@@ -190,3 +190,26 @@ def test_wide_inputs_in_several_launches(gpu, I, H, L, B, T, lengths):
     want = _oracle(native, few, lengths=lens.numpy() if lengths else None)
     assert np.abs(res["out_seq"][:3].float().cpu().numpy() - want["out_seq"]).max() <= 2 * BOUND
     assert np.abs(res["h_n"][:, :3].float().cpu().numpy() - want["h_n"]).max() <= 2 * BOUND
+
+
+@pytest.mark.parametrize("I,H,L,B,T,same", [
+    (5, 400, 4, 740, 12, True),    # 512 rows and 228, which four launches would take: layer by layer too
+    (5, 512, 2, 700, 9, True),     # ... two launches of the sliced kernel
+    (5, 300, 3, 740, 20, True),
+    (100, 512, 4, 560, 12, False),  # one launch: all layers at once (projections of layers >= 1 in fp32)
+])
+def test_path_of_the_rows_after_a_layer_sequential_launch(gpu, I, H, L, B, T, same):
+    """Padded H 512: the rows after the last full launch change to the sliced kernel only where that is faster.
+    Elsewhere all rows are computed alike, so equal rows are equal bit for bit; the oracle's bound holds for both."""
+    print(f"[gpu-case] H512 remainder I={I} H={H} L={L} B={B} T={T}", flush=True)
+    native = make_regressor(I, H, L, 3)
+    few = make_x(3, T, I, seed=7)
+    which = torch.arange(B) % 3
+    out, (h, c) = _lstm(native)(few.to("cuda", torch.float16)[which.cuda()])
+    gpu.check_status(torch.device("cuda"))
+    alike = torch.equal(out, out[:3][which.cuda()]) and torch.equal(c, c[:, :3][:, which.cuda()])
+    assert alike == same
+    want = _oracle(native, few)
+    ends = np.r_[0:3, B - 3:B]
+    assert np.abs(out[ends].float().cpu().numpy() - want["out_seq"][ends % 3]).max() <= 2 * BOUND
+    assert np.abs(h[:, ends].float().cpu().numpy() - want["h_n"][:, ends % 3]).max() <= 2 * BOUND
