@@ -538,11 +538,17 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
   // ---- steps ----
   // Step t, for both tiles of a two-tile workgroup at once (the exchange's round trip, the memory
   // issue and the barrier are paid once per step, not per tile): h_{t-1} W_hh^T; each tile's cell
-  // update, output sequence and word; each tile's input part x_{t+1} W_ih^T (the last step computes a
-  // discarded one) with the polls of step t inside it; the gathers into the other h buffer; then,
+  // update, output sequence and word; each tile's input part x_{t+1} W_ih^T (the last step may compute
+  // a discarded one) with the polls of step t inside it; the gathers into the other h buffer; then,
   // off the step's chain, the input of step t + 2 into the ring, the hand-off copy of h_{t-1}, the
   // input pieces of step t + 3 and the counter (issued after the gathers, so that no wait of this
   // step covers them); one barrier, after which thread 0 publishes.
+  // One tile at padded H 256: each half of the input part stands in a branch of its own (the last step skips it), a
+  // region that the compiler schedules by itself.  Without the branches a launch of few groups (layers of a tile
+  // on different XCDs) was slower than with its polls behind the whole input part: T 200, polls behind -> without
+  // -> with, L2 B8 311 -> 313 -> 291 us, L4 B8 342 -> 349 -> 337, L4 B32 338 -> 354 -> 344, L8 B8 392 -> 404 -> 392; L1 B64
+  // 283 -> 267 -> 266, L4 B128 344 -> 328 -> 323.  At H 512 and with two tiles the branches cost 1-3%.
+  constexpr bool kGuardInput = NTI == 1 && HP == 256;
   for (int t = 0; ok && t < Tt; ++t) {
 #pragma unroll
     for (int i = 0; i < NTI; ++i) rec_mfma(i, hbuf[i][t & 1]);
@@ -554,11 +560,12 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < NTI; ++i) {
-      input_mfma(i, t + 1, Chunk<0>(), Chunk<kPollChunk>());
+      const bool next = !kGuardInput || t + 1 < Tt;
+      if (next) input_mfma(i, t + 1, Chunk<0>(), Chunk<kPollChunk>());
       __builtin_amdgcn_sched_barrier(0);
       issue_poll(i, t);
       __builtin_amdgcn_sched_barrier(0);
-      input_mfma(i, t + 1, Chunk<kPollChunk>(), Chunk<KCH>());
+      if (next) input_mfma(i, t + 1, Chunk<kPollChunk>(), Chunk<KCH>());
     }
 #pragma unroll
     for (int i = 0; i < NTI; ++i) gather(i, t, hbuf[i][(t + 1) & 1]);
