@@ -538,11 +538,13 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
   // ---- steps ----
   // Step t, for both tiles of a two-tile workgroup at once (the exchange's round trip, the memory
   // issue and the barrier are paid once per step, not per tile): h_{t-1} W_hh^T; each tile's cell
-  // update, output sequence and word; each tile's input part x_{t+1} W_ih^T (the last step may compute
-  // a discarded one) with the polls of step t inside it; the gathers into the other h buffer; then,
-  // off the step's chain, the input of step t + 2 into the ring, the hand-off copy of h_{t-1}, the
-  // input pieces of step t + 3 and the counter (issued after the gathers, so that no wait of this
-  // step covers them); one barrier, after which thread 0 publishes.
+  // update and word; each tile's input part x_{t+1} W_ih^T (the last step may compute a discarded
+  // one) with the polls of step t inside it; the gathers into the other h buffer; then, off the
+  // step's chain, the output sequence, the input of step t + 2 into the ring, the hand-off copy of
+  // h_{t-1}, the input pieces of step t + 3 and the counter (issued after the gathers, so that no wait
+  // of this step covers them); one barrier, after which thread 0 publishes.
+  // (The output sequence, stored in front of the word, had to complete before the polls behind it: T 200, L1 B64
+  // H 256 with a sequence 317 -> 284 us, L4 B128 360 -> 327, H400 L2 B40 T128 254 -> 239.)
   // One tile at padded H 256: each half of the input part stands in a branch of its own (the last step skips it), a
   // region that the compiler schedules by itself.  Without the branches a launch of few groups (layers of a tile
   // on different XCDs) was slower than with its polls behind the whole input part: T 200, polls behind -> without
@@ -555,7 +557,6 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
 #pragma unroll
     for (int i = 0; i < NTI; ++i) {
       cell(i, t);
-      store_out_seq(i, t);
       send(i, t);
     }
 #pragma unroll
@@ -572,6 +573,7 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
 #pragma unroll
     for (int i = 0; i < NTI; ++i) {
       settle(i);
+      store_out_seq(i, t);
       store_piece(i, t + 2);
       if (t > 0) copy_out(i, t - 1, hbuf[i][t & 1]);
       if (threadIdx.x == 0) s_up[i] = cup[i];

@@ -18,6 +18,7 @@ from __future__ import annotations
 import os
 import weakref
 from functools import lru_cache
+from operator import itemgetter
 from typing import Any, Optional, Sequence, Tuple
 
 import torch
@@ -122,10 +123,11 @@ class _TensorSetKey:
 
 
 @lru_cache(maxsize=None)
-def _param_names(num_layers: int, bias: bool) -> Tuple[str, ...]:
-    """The attributes that PersistentLSTM packs, layer by layer."""
+def _param_getter(num_layers: int, bias: bool) -> itemgetter:
+    """Takes the tensors that PersistentLSTM packs out of its parameter table, layer by layer (KeyError if one of
+    them is not there)."""
     kinds = ("weight_ih", "weight_hh", "bias_ih", "bias_hh") if bias else ("weight_ih", "weight_hh")
-    return tuple(f"{kind}_l{l}" for l in range(num_layers) for kind in kinds)
+    return itemgetter(*(f"{kind}_l{l}" for l in range(num_layers) for kind in kinds))
 
 
 class PersistentLSTM(nn.Module):
@@ -182,11 +184,10 @@ class PersistentLSTM(nn.Module):
         them is a parameter under its own name (an attribute look-up each costs several times that), else, for
         a weight that something else computes from a parameter of another name (pruning, a spectral or weight
         norm, a parametrization), through the attributes."""
-        own = self._parameters
         try:
-            params = [own[name] for name in _param_names(self.num_layers, self.bias)]
+            params = _param_getter(self.num_layers, self.bias)(self._parameters)
         except KeyError:
-            params = [p for l in range(self.num_layers) for p in self.layer_params(l)]
+            params = tuple(p for l in range(self.num_layers) for p in self.layer_params(l))
         if linear is not None:
             params += (linear.weight, linear.bias)
         dev = (device.type, device.index)
