@@ -12,7 +12,7 @@
 //   * weight-stationary: each workgroup owns one 128-column slice of W, loaded once into LDS in MFMA
 //     fragment order when K <= 512 (for K > 512 the slice is held in K blocks that take turns in LDS
 //     for every m-tile, between two barriers: of 512 in proj_gemm_kernel, of 256 or 128 with the first
-//     ones kept in proj_gemm_blocked_kernel), and walks the 512-row m-tiles of its m-group; its
+//     one kept in proj_gemm_blocked_kernel), and walks the 512-row m-tiles of its m-group; its
 //     8 waves (two per SIMD) each compute a 64 (m) x 128 (n) sub-tile with v_mfma_f32_16x16x32_f16
 //     (4 x 8 accumulator tiles, 128 fp32 per lane), W as the MFMA's A operand and X as its B operand;
 //   * X goes from global memory straight into the B-fragment registers (a lane's 8 consecutive k
@@ -219,28 +219,27 @@ proj_gemm_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* 
 // (interleaved runs on one box each); the stores in the next tile's first step: 0.943-0.951 ->
 // 0.933-0.935 ms and 0.105-0.106 -> 0.104-0.106 ms, bit-identical.
 //
-// MULTI: the W slice does not fit the LDS.  Its first KEEP blocks stay there (K = 1024: one of 256; odd multiples of
-// 128: three of 128), the others are reloaded for every tile, from global memory to LDS directly (16 bytes per
-// lane, no registers).  Every tile takes its blocks in ascending order, so a row's sums do not depend on the
-// tile it stands in: equal rows have equal results, and the bits are those of the run-time-K kernel.  (Walking
-// the blocks up and down, with the block left by one tile the next one's first, reloads as many blocks of 256
-// but summed odd and even tiles in opposite orders; reloading all of them in ascending order took 1.02, 0.79
-// and 0.64 ms where the alternation took 0.93, 0.69 and 0.61.)  Interleaved on one box, the alternation -> this:
-// [128000,1024]x[1024,4096] 0.985-0.999 -> 0.996-1.003 ms, K = 768 0.732-0.734 -> 0.729-0.731, K = 640 0.641-0.643
-// -> 0.572-0.573; the run-time-K kernel, which reloads blocks of 512 twice per tile: 1.06, 0.82 and 0.71 on a
-// box where the alternation took 0.93, 0.69 and 0.61.  Blocks of 512 spilled 21 VGPRs (+3%); two buffers, the
-// next block loading under the current one's MFMAs, were 2-6% slower.
+// MULTI: the W slice does not fit the LDS.  Its first block stays there, the others are reloaded for every tile,
+// from global memory to LDS directly (16 bytes per lane, no registers).  Every tile takes its blocks in
+// ascending order, so a row's sums do not depend on the tile it stands in: equal rows have equal results, and
+// the bits are those of the run-time-K kernel.  (Walking the blocks up and down, with the block left by one tile
+// the next one's first, reloads as many but summed odd and even tiles in opposite orders; reloading all of them
+// in ascending order took 1.02, 0.79 and 0.64 ms where the walk took 0.93, 0.69 and 0.61.)  Interleaved on one box,
+// the walk -> this: [128000,1024]x[1024,4096] 0.915-0.923 -> 0.918-0.920 ms, K = 768 0.681-0.683 -> 0.678-0.681,
+// K = 640 0.598-0.601 -> 0.607-0.612; the run-time-K kernel, which reloads blocks of 512 twice per tile: 1.06, 0.82
+// and 0.71 on a box where the walk took 0.93, 0.69 and 0.61.  Keeping three blocks of 128: K = 640 0.57 ms, but
+// on boxes at their power limit the recurrent kernels beside it slowed by more (H 784 L8 B103: 2.05 -> 2.10-2.20
+// ms).  Blocks of 512 spilled 21 VGPRs (+3%); two buffers, the next block loading under the current one's
+// MFMAs, were 2-6% slower.
 template <int KS, bool MULTI>
 __global__ void __launch_bounds__(kGemmThreads)
 proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _Float16* __restrict__ W, int blocks,
                          _Float16* __restrict__ C, long long ldc, int M, int tiles_m, int n_slices, int m_groups) {
   static_assert(kGemmWaves == 8 && kGemmWM == 4 && KS % kRing == 0 && KS * 32 <= kGemmMaxK, "tile shape");
   const int K = MULTI ? 32 * KS * blocks : 32 * KS;
-  // MULTI: blocks 0 .. KEEP - 1 stay in LDS for good (slots 1 .. KEEP), the others take turns in slot 0.
-  constexpr int KEEP = MULTI ? kGemmKbSteps / KS - 1 : 0;
-  static_assert(!MULTI || KEEP >= 1, "a tile's first block is one that stays");
+  // MULTI: block 0 stays in LDS for good (slot 1), the others take turns in slot 0.
   constexpr int kSlotVec = KS * 8 * 64;  // f16x8 of one block: [k-chunk][n-tile 0..7][64 lanes]
-  __shared__ f16x8 wl[(KEEP + 1) * kSlotVec];
+  __shared__ f16x8 wl[(MULTI ? 2 : 1) * kSlotVec];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   const int ns = idx % n_slices;
@@ -263,8 +262,7 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
     }
     if constexpr (decltype(direct)::value) wait_vmem_all();
   };
-#pragma unroll
-  for (int b = 0; b < (MULTI ? KEEP : 1); ++b) load_w(b, MULTI ? 1 + b : 0, std::false_type());
+  load_w(0, MULTI ? 1 : 0, std::false_type());
   __syncthreads();
   int mt = mg;
   if (mt >= tiles_m) return;
@@ -308,7 +306,7 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
   auto kstep = [&](int s, int kb, __amdgpu_buffer_rsrc_t rc, __amdgpu_buffer_rsrc_t rn, int nb,
                    const __amdgpu_buffer_rsrc_t* out) __attribute__((always_inline)) {
     const bool first = kb == 0;
-    const f16x8* const wk = wl + (kb < KEEP ? 1 + kb : 0) * kSlotVec + lane;
+    const f16x8* const wk = wl + (MULTI && kb == 0 ? kSlotVec : 0) + lane;
     __builtin_amdgcn_sched_barrier(0);
     {
       const int sn = s + kRing - 1;  // this tile's step sn, or the next tile's first steps
@@ -393,12 +391,10 @@ proj_gemm_blocked_kernel(const _Float16* __restrict__ X, long long ldx, const _F
     if constexpr (MULTI) {
 #pragma unroll 1
       for (int kb = 1; kb < blocks; ++kb) {
-        if (kb >= KEEP) {
-          // every wave is done with the slot (its MFMAs read it from registers loaded before them)
-          __syncthreads();
-          load_w(kb, 0, std::true_type());
-          __syncthreads();
-        }
+        // every wave is done with the slot (its MFMAs read it from registers loaded before them)
+        __syncthreads();
+        load_w(kb, 0, std::true_type());
+        __syncthreads();
         const bool more = kb + 1 < blocks;
         const auto rx = more ? rc : rn;
         const int nb = more ? kb + 1 : 0;
