@@ -544,12 +544,13 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
   // h_{t-1}, the input pieces of step t + 3 and the counter (issued after the gathers, so that no wait
   // of this step covers them); one barrier, after which thread 0 publishes.
   // (The output sequence, stored in front of the word, had to complete before the polls behind it: T 200, L1 B64
-  // H 256 with a sequence 317 -> 284 us, L4 B128 360 -> 327, H400 L2 B40 T128 254 -> 239.)
+  // H 256 with a sequence 317 -> 284 us, L4 B128 360 -> 327, H400 L2 B40 T128 254 -> 239.  Two tiles keep it there:
+  // behind the gathers it gave 4% with a sequence and cost 0.5-1% without one.)
   // One tile at padded H 256: each half of the input part stands in a branch of its own (the last step skips it), a
   // region that the compiler schedules by itself.  Without the branches a launch of few groups (layers of a tile
   // on different XCDs) was slower than with its polls behind the whole input part: T 200, polls behind -> without
-  // -> with, L2 B8 311 -> 313 -> 291 us, L4 B8 342 -> 349 -> 337, L4 B32 338 -> 354 -> 344, L8 B8 392 -> 404 -> 392; L1 B64
-  // 283 -> 267 -> 266, L4 B128 344 -> 328 -> 323.  At H 512 and with two tiles the branches cost 1-3%.
+  // -> with, L2 B8 311 -> 313 -> 291 us, L4 B8 342 -> 349 -> 337, L4 B32 338 -> 354 -> 344, L8 B8 392 -> 404 -> 392;
+  // L1 B64 283 -> 267 -> 266, L4 B128 344 -> 328 -> 323.  At H 512 and with two tiles the branches cost 1-3%.
   constexpr bool kGuardInput = NTI == 1 && HP == 256;
   for (int t = 0; ok && t < Tt; ++t) {
 #pragma unroll
@@ -557,23 +558,31 @@ __global__ void __launch_bounds__(512) lstm_sliced_kernel(ForwardArgs a) {
 #pragma unroll
     for (int i = 0; i < NTI; ++i) {
       cell(i, t);
+      if constexpr (NTI == 2) store_out_seq(i, t);
       send(i, t);
     }
 #pragma unroll
     for (int i = 0; i < NTI; ++i) {
-      const bool next = !kGuardInput || t + 1 < Tt;
-      if (next) input_mfma(i, t + 1, Chunk<0>(), Chunk<kPollChunk>());
+      if constexpr (kGuardInput) {
+        if (t + 1 < Tt) input_mfma(i, t + 1, Chunk<0>(), Chunk<kPollChunk>());
+      } else {
+        input_mfma(i, t + 1, Chunk<0>(), Chunk<kPollChunk>());
+      }
       __builtin_amdgcn_sched_barrier(0);
       issue_poll(i, t);
       __builtin_amdgcn_sched_barrier(0);
-      if (next) input_mfma(i, t + 1, Chunk<kPollChunk>(), Chunk<KCH>());
+      if constexpr (kGuardInput) {
+        if (t + 1 < Tt) input_mfma(i, t + 1, Chunk<kPollChunk>(), Chunk<KCH>());
+      } else {
+        input_mfma(i, t + 1, Chunk<kPollChunk>(), Chunk<KCH>());
+      }
     }
 #pragma unroll
     for (int i = 0; i < NTI; ++i) gather(i, t, hbuf[i][(t + 1) & 1]);
 #pragma unroll
     for (int i = 0; i < NTI; ++i) {
       settle(i);
-      store_out_seq(i, t);
+      if constexpr (NTI == 1) store_out_seq(i, t);
       store_piece(i, t + 2);
       if (t > 0) copy_out(i, t - 1, hbuf[i][t & 1]);
       if (threadIdx.x == 0) s_up[i] = cup[i];
