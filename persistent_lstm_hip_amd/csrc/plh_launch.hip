@@ -25,8 +25,9 @@ bool make_geometry(int I, int H, int L, int O, Geometry* g, std::string* why) {
   }
   int HP = H <= 32 ? 32 : H <= 64 ? 64 : H <= 128 ? 128 : H <= 256 ? 256 : H <= 512 ? 512 : 1024;
   // An input wider than the padded hidden size does not fit the all-layers kernels' resident input
-  // part: such a model runs layer by layer (its layer-0 projection a GEMM over any K), whose kernels
-  // start at padded H 128 (the extra padded units stay exactly zero).
+  // part: layer 0's projection is a GEMM over any K, in front of the wavefront kernel (padded H 128, see plan_for)
+  // or of the layer-sequential path, whose kernels start at padded H 128 (the extra padded units stay exactly
+  // zero).
   if (I > HP && HP < 128) HP = 128;
   g->I = I;
   g->H = H;
